@@ -54,6 +54,10 @@ using namespace boids;
 
 static thread_local std::string g_create_error;
 
+// Largest metrics workspace an engine keeps for its next call (flocks of up
+// to ~10^6 boids); a larger one is allocated and released inside the call.
+constexpr size_t kMetricsKeep = (size_t)64 << 20;
+
 // Static device scratch of the allocation-free entry point
 // (bs_metrics_flock_noalloc): kScratchBytes on every GPU the library runs
 // on, held until the process ends.  On the host, `scratch` names a host-side
@@ -137,6 +141,8 @@ struct bs_engine {
     void* forces = nullptr;   // float or double, 9n, id order
     uint64_t* digest = nullptr;
     double *tmp_pos = nullptr, *tmp_vel = nullptr;
+    void* metrics_ws = nullptr;        // kept between metrics calls (at most kMetricsKeep)
+    size_t metrics_ws_bytes = 0;
 
     // timing
     struct Pending { int kernel; hipEvent_t a, b; };
@@ -548,6 +554,7 @@ static void release(bs_engine* e)
     for (auto& p : e->pending) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
     for (auto ev : e->free_events) (void)hipEventDestroy(ev);
     if (e->graph) (void)hipGraphExecDestroy(e->graph);
+    if (e->metrics_ws) (void)hipFree(e->metrics_ws);
     for (void* p : e->allocs) (void)hipFree(p);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     delete e;
@@ -1290,8 +1297,9 @@ extern "C" int bs_debug_copy(uint64_t bytes, int32_t reps, double* ms_per_copy)
 }
 
 // Flock metrics of the current state (see boids_metrics.hip).  The
-// workspace is temporary device memory allocated and released inside the
-// call, or (static_ws) the device's static scratch array.  Flock k of a
+// workspace is the engine's (grown when a call needs more, temporary beyond
+// kMetricsKeep: allocating and releasing it took a third of a call at
+// 131072 boids), or (static_ws) the device's static scratch array.  Flock k of a
 // batch is the id range [boid_base, boid_base + n) of the unsorted state.
 static int metrics_impl(bs_engine* e, uint32_t flock, double eps, uint32_t min_size, bs_metrics_out* out,
                         bool static_ws)
@@ -1307,14 +1315,16 @@ static int metrics_impl(bs_engine* e, uint32_t flock, double eps, uint32_t min_s
     const double F = e->flocks.empty() ? e->prm.field : e->flock_field[flock];
     memset(out, 0, sizeof(*out));
     if (n == 0) return BS_OK;
-    // edge >= eps (links need only the 27 neighbouring cells); no more cells than ~8 per boid
-    double g = eps > 0.0 ? floor(F / (eps * 1.0001)) : 1024.0;
-    const double cap = std::max(1.0, 2.0 * floor(cbrt((double)n)));
-    g = std::min(std::min(g, cap), 1024.0);
-    const int G = std::max(1, (int)g);
+    // edge >= eps (links need only the 27 neighbouring cells); no more cells than
+    // boids: eight per boid, as the static scratch is still priced, left most
+    // searches for a third ring of 98 cells
+    const double root = floor(cbrt((double)n));
+    const double most = std::min(eps > 0.0 ? floor(F / (eps * 1.0001)) : 1024.0, 1024.0);
+    const int G = std::max(1, (int)std::min(most, std::max(1.0, root)));
     const size_t bytes = metrics_workspace_bytes(n, G);
-    if (static_ws && bytes > kScratchBytes)
-        return fail(e, BS_E_ARG, "metrics workspace of " + std::to_string(bytes) + " bytes exceeds the static scratch (" +
+    const size_t priced = metrics_priced_bytes(n, std::max(1, (int)std::min(most, std::max(1.0, 2.0 * root))));
+    if (static_ws && priced > kScratchBytes)
+        return fail(e, BS_E_ARG, "metrics workspace of " + std::to_string(priced) + " bytes exceeds the static scratch (" +
                                      std::to_string(kScratchBytes) + " bytes): use bs_metrics_flock");
     if (static_ws && !e->scratch) return fail(e, BS_E_STATE, "static scratch unavailable: " + e->scratch_why);
     if (is_f32(e->mode))
@@ -1322,16 +1332,34 @@ static int metrics_impl(bs_engine* e, uint32_t flock, double eps, uint32_t min_s
     else
         HIP_TRY(e, launch_unsort_f64(ntot, e->da, e->tmp_pos, e->tmp_vel, e->stream));
     void* ws = nullptr;
-    if (static_ws) ws = e->scratch;
-    else if (hipMalloc(&ws, bytes) != hipSuccess) return fail(e, BS_E_NOMEM, "metrics workspace allocation failed");
+    const bool keep = !static_ws && bytes <= kMetricsKeep;
+    if (static_ws) {
+        ws = e->scratch;
+    } else if (keep && e->metrics_ws_bytes >= bytes) {
+        ws = e->metrics_ws;
+    } else {
+        if (keep && e->metrics_ws) {           // too small: grow (calls end synchronised, so it is idle)
+            (void)hipFree(e->metrics_ws);
+            e->device_bytes -= e->metrics_ws_bytes;
+            e->metrics_ws = nullptr;
+            e->metrics_ws_bytes = 0;
+        }
+        if (hipMalloc(&ws, bytes) != hipSuccess) return fail(e, BS_E_NOMEM, "metrics workspace allocation failed");
+        if (keep) {
+            e->metrics_ws = ws;
+            e->metrics_ws_bytes = bytes;
+            e->device_bytes += bytes;
+        }
+    }
     double* res = nullptr;
     hipError_t st = launch_metrics(n, F, G, eps, min_size, e->tmp_pos + 3 * (size_t)base,
-                                   e->tmp_vel + 3 * (size_t)base, ws, static_ws ? kScratchBytes : bytes, &res,
+                                   e->tmp_vel + 3 * (size_t)base, ws, static_ws ? kScratchBytes : (keep ? e->metrics_ws_bytes : bytes), &res,
                                    e->stream);
     double host[4] = {0, 0, 0, 0};
     if (st == hipSuccess) st = hipMemcpyAsync(host, res, sizeof(host), hipMemcpyDeviceToHost, e->stream);
     if (st == hipSuccess) st = hipStreamSynchronize(e->stream);
-    if (!static_ws) (void)hipFree(ws);
+    if (st != hipSuccess) (void)hipStreamSynchronize(e->stream);   // nothing may run on the workspace any more
+    if (!static_ws && !keep) (void)hipFree(ws);
     if (st != hipSuccess) return hip_fail(e, st, "metrics");
     out->polarisation = host[0];
     out->mean_nn = host[1];

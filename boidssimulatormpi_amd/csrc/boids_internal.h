@@ -121,8 +121,6 @@ hipError_t launch_scan(uint32_t* count, uint32_t* start, uint32_t n, uint32_t* p
 hipError_t launch_rows(Flocks F, const uint32_t* start, uint32_t* row_count, uint32_t* row_off,
                        uint32_t* partials, uint4* table, uint32_t* nchunks, uint32_t cap, uint32_t* overflow,
                        int chunk, int cspan, int max_cols, hipStream_t stream);
-hipError_t launch_scatter(uint32_t n, const uint32_t* key, const uint32_t* start, uint32_t* count,
-                          const uint32_t* id, uint32_t* perm, uint32_t* permid, hipStream_t stream);
 // Scatter by the arrival ranks the counting pass recorded (no atomics),
 // then sort every run of 64 slots by (cell, id) (the gather merges a cell's
 // sorted parts into its in-cell id order).
@@ -162,6 +160,10 @@ hipError_t launch_f32_grid_step(const DevParams& P, StateF32 in, StateF32 out, c
                                 uint64_t* digest, hipStream_t stream);
 // flock metrics (boids_metrics.hip)
 size_t metrics_workspace_bytes(uint32_t n, int G);
+// What the static scratch is priced at: 64 bytes per boid and 8 per cell of a
+// G-cell grid, in 256-byte regions.  A flock beyond the scratch at this price
+// is refused there, though its workspace takes less by now.
+size_t metrics_priced_bytes(uint32_t n, int G);
 // Workspace regions are carved from `ws` (metrics_workspace_bytes long);
 // *out4_dev receives the device address of the 4 result doubles.
 hipError_t launch_metrics(uint32_t n, double F, int G, double eps, uint32_t min_size, const double* pos3,

@@ -159,7 +159,7 @@ constexpr int kScanItems = 4;
 constexpr int kScanTile = kScanThreads * kScanItems;
 
 // Tile-local exclusive scan of count[] into start[]; tile totals into
-// partials[]; count[] is cleared for reuse as the scatter's fill counter.
+// partials[]; count[] is cleared for the next update's counts.
 __global__ __launch_bounds__(kScanThreads) void k_scan_tiles(uint32_t* count, uint32_t* start,
                                                               uint32_t m, uint32_t* partials)
 {
@@ -276,19 +276,6 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_rows_pass(Flocks F, const ui
         }
     }
     if (!WRITE) row_count[r] = k;
-}
-
-__global__ __launch_bounds__(kBlock) void k_scatter(uint32_t n, const uint32_t* key,
-                                                    const uint32_t* start, uint32_t* count,
-                                                    const uint32_t* id, uint32_t* perm,
-                                                    uint32_t* permid)
-{
-    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
-    if (s >= n) return;
-    const uint32_t c = key[s];
-    const uint32_t t = start[c] + atomicAdd(&count[c], 1u);
-    perm[t] = s;
-    permid[t] = id[s];
 }
 
 __global__ __launch_bounds__(kBlock) void k_scatter_ranked(uint32_t n, const uint32_t* __restrict__ key,
@@ -483,15 +470,6 @@ hipError_t launch_rows(Flocks F, const uint32_t* start, uint32_t* row_count, uin
     hipLaunchKernelGGL(k_rows_pass<true>, grid, dim3(64 * kRowWaves), dyn, stream, F, start, row_count,
                        (const uint32_t*)row_off, table, nchunks, (uint32_t)chunk, (uint32_t)cspan, stride, cap,
                        overflow);
-    return hipGetLastError();
-}
-
-hipError_t launch_scatter(uint32_t n, const uint32_t* key, const uint32_t* start, uint32_t* count,
-                          const uint32_t* id, uint32_t* perm, uint32_t* permid, hipStream_t stream)
-{
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_scatter, dim3(blocks_for(n)), dim3(kBlock), 0, stream, n, key, start,
-                       count, id, perm, permid);
     return hipGetLastError();
 }
 

@@ -245,9 +245,10 @@ int bs_metrics_flock(bs_engine* e, uint32_t flock, double eps, uint32_t min_size
  * reference: it is for callers that cannot allocate (analysis inside tight
  * stepping loops, harnesses that forbid hipMalloc).  Its workspace is a
  * static device array of 64 MiB on every GPU the library runs on (held
- * until the process ends) instead of temporary memory; a flock whose
- * workspace exceeds it is rejected with BS_E_ARG (the workspace takes at
- * most ~128 bytes per boid: flocks of up to ~5 x 10^5 boids always fit).
+ * until the process ends) instead of the engine's own workspace (which
+ * bs_metrics and bs_metrics_flock keep between calls up to 64 MiB, and
+ * otherwise release at once); a flock priced above it, at ~128 bytes per
+ * boid, is rejected with BS_E_ARG (up to ~5 x 10^5 boids always fit).
  * Every call on one GPU shares that array: calls that overlap on one GPU
  * race.  Results equal bs_metrics_flock's. */
 int bs_metrics_flock_noalloc(bs_engine* e, uint32_t flock, double eps, uint32_t min_size, bs_metrics_out* out);
