@@ -41,13 +41,17 @@ static_assert(BS_MIXED_CHUNK_SPAN >= 1 && BS_MIXED_CHUNK_SPAN <= boids::kChunkSp
 #include <math.h>
 #include <stdio.h>
 #include <string.h>
+#include <sys/mman.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdint>
 #include <fstream>
 #include <map>
 #include <mutex>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 using namespace boids;
@@ -85,6 +89,72 @@ static void* scratch_address(int device, std::string* why)
     }
     g_scratch_addr[device] = ptr;
     return ptr;
+}
+
+// Pinned staging buffers of the state and force transfers, lent to one call at
+// a time (several threads may hold one each).  Buffers that come back are
+// kept for the next call, at most kStageKept of them, and released with the
+// last engine: allocating pinned memory takes about 0.3 ms per MB.
+constexpr size_t kStageKept = 4;
+struct StageBuf { char* p; size_t bytes; };
+static std::mutex g_stage_mu;
+static StageBuf g_stage_free[kStageKept];
+static size_t g_stage_count = 0, g_stage_engines = 0;
+
+static char* stage_take(size_t want, size_t* bytes)
+{
+    {
+        std::lock_guard<std::mutex> lk(g_stage_mu);
+        for (size_t k = 0; k < g_stage_count; ++k)
+            if (g_stage_free[k].bytes >= want) {
+                const StageBuf b = g_stage_free[k];
+                g_stage_free[k] = g_stage_free[--g_stage_count];
+                *bytes = b.bytes;
+                return b.p;
+            }
+    }
+    size_t size = (size_t)1 << 16;
+    while (size < want) size <<= 1;
+    void* p = nullptr;
+    if (hipHostMalloc(&p, size, hipHostMallocPortable) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+    *bytes = size;
+    return (char*)p;
+}
+
+static void stage_back(char* p, size_t bytes)
+{
+    if (!p) return;
+    {
+        std::lock_guard<std::mutex> lk(g_stage_mu);
+        if (g_stage_engines && g_stage_count < kStageKept) {
+            g_stage_free[g_stage_count++] = {p, bytes};
+            return;
+        }
+        if (g_stage_engines)                       // full: keep the larger ones
+            for (auto& f : g_stage_free)
+                if (f.bytes < bytes) { std::swap(f.p, p); std::swap(f.bytes, bytes); break; }
+    }
+    (void)hipHostFree(p);
+}
+
+static void stage_engine_created()
+{
+    std::lock_guard<std::mutex> lk(g_stage_mu);
+    ++g_stage_engines;
+}
+
+static void stage_engine_gone()
+{
+    StageBuf gone[kStageKept];
+    size_t count = 0;
+    {
+        std::lock_guard<std::mutex> lk(g_stage_mu);
+        if (--g_stage_engines == 0) {
+            std::copy(g_stage_free, g_stage_free + g_stage_count, gone);
+            std::swap(count, g_stage_count);
+        }
+    }
+    for (size_t k = 0; k < count; ++k) (void)hipHostFree(gone[k].p);
 }
 
 struct bs_engine {
@@ -134,13 +204,15 @@ struct bs_engine {
     double2* rec = nullptr;            // FP64 grid: interleaved pair records
     float4 *rec4 = nullptr, *vrec4 = nullptr;   // float grid: sorted positions (+ id) and velocities
     uint32_t* recheck = nullptr;
-    uint32_t* overflow = nullptr;      // chunk-table count beyond its capacity (0: none)
+    uint32_t* overflow = nullptr;      // chunk-table count beyond its capacity (0: none), in pinned host memory
     void* scratch = nullptr;           // this device's static scratch (allocation-free entry points)
     std::string scratch_why;           // why it is unavailable
     // outputs
     void* forces = nullptr;   // float or double, 9n, id order
     uint64_t* digest = nullptr;
     double *tmp_pos = nullptr, *tmp_vel = nullptr;
+    hipEvent_t stage_ev[8] = {nullptr};   // one per thread of a transfer
+    bool counted = false;                 // among the staging pool's engines
     void* metrics_ws = nullptr;        // kept between metrics calls (at most kMetricsKeep)
     size_t metrics_ws_bytes = 0;
 
@@ -554,9 +626,13 @@ static void release(bs_engine* e)
     for (auto& p : e->pending) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
     for (auto ev : e->free_events) (void)hipEventDestroy(ev);
     if (e->graph) (void)hipGraphExecDestroy(e->graph);
+    for (auto ev : e->stage_ev)
+        if (ev) (void)hipEventDestroy(ev);
+    if (e->overflow) (void)hipHostFree(e->overflow);
     if (e->metrics_ws) (void)hipFree(e->metrics_ws);
     for (void* p : e->allocs) (void)hipFree(p);
     if (e->stream) (void)hipStreamDestroy(e->stream);
+    if (e->counted) stage_engine_gone();
     delete e;
 }
 
@@ -742,7 +818,8 @@ static int create_engine(const bs_params* fp, uint32_t count, bool batch, bs_eng
         if (e->mode == BS_MODE_ALLPAIRS_F64) e->db.id = e->da.id;   // all-pairs stays in id order
         if (p->flags & BS_FLAG_FORCES) { double* f; if ((rc = dev_alloc(e, &f, 9 * (size_t)n))) return bail(rc); e->forces = f; }
     }
-    if ((rc = dev_alloc(e, &e->tmp_pos, 3 * (size_t)n)) || (rc = dev_alloc(e, &e->tmp_vel, 3 * (size_t)n))) return bail(rc);
+    if ((rc = dev_alloc(e, &e->tmp_pos, 6 * (size_t)n))) return bail(rc);
+    e->tmp_vel = e->tmp_pos + 3 * (size_t)n;
     if (p->flags & BS_FLAG_DIGEST) { if ((rc = dev_alloc(e, &e->digest, 4 * (size_t)n))) return bail(rc); }
     if (e->mode == BS_MODE_GRID_F32REF) {
         const uint32_t ntiles = (e->ncell1 + 4095) / 4096;
@@ -764,7 +841,6 @@ static int create_engine(const bs_params* fp, uint32_t count, bool batch, bs_eng
             (rc = dev_alloc(e, &e->partials, ntiles)) || (rc = dev_alloc(e, &e->nchunks, 1)) ||
             (rc = dev_alloc(e, &e->perm, n)) || (rc = dev_alloc(e, &e->permid, n)) || (rc = dev_alloc(e, &e->rank, n)) ||
             (rc = dev_alloc(e, &e->table, e->max_chunks)) || (rc = dev_alloc(e, &e->recheck, 1)) ||
-            (rc = dev_alloc(e, &e->overflow, 1)) ||
             (rc = dev_alloc(e, &e->row_count, (size_t)e->rows + 1)) ||
             (rc = dev_alloc(e, &e->row_off, (size_t)e->rows + 1)) ||
             (rc = dev_alloc(e, &e->flocks_dev, e->flocks.size())))
@@ -791,9 +867,14 @@ static int create_engine(const bs_params* fp, uint32_t count, bool batch, bs_eng
         } else if ((rc = dev_alloc(e, &e->rec, 3 * (size_t)n))) {
             return bail(rc);
         }
+        // written by the device only when a table overflows, read by the host after a synchronisation: no copy
+        void* word = nullptr;
+        st = hipHostMalloc(&word, sizeof(uint32_t), hipHostMallocDefault);
+        if (st != hipSuccess) return bail(fail(e, BS_E_NOMEM, "hipHostMalloc failed"));
+        e->overflow = (uint32_t*)word;
+        *e->overflow = 0;
         st = hipMemsetAsync(e->count, 0, sizeof(uint32_t) * e->ncell1, e->stream);
         if (st == hipSuccess) st = hipMemsetAsync(e->recheck, 0, sizeof(uint32_t), e->stream);
-        if (st == hipSuccess) st = hipMemsetAsync(e->overflow, 0, sizeof(uint32_t), e->stream);
         if (st != hipSuccess) { hip_fail(e, st, "hipMemsetAsync"); return bail(BS_E_HIP); }
     }
     if (e->forces) {
@@ -807,6 +888,8 @@ static int create_engine(const bs_params* fp, uint32_t count, bool batch, bs_eng
     }
     st = hipStreamSynchronize(e->stream);
     if (st != hipSuccess) { hip_fail(e, st, "hipStreamSynchronize"); return bail(BS_E_HIP); }
+    stage_engine_created();
+    e->counted = true;
     *out = e;
     return BS_OK;
 }
@@ -887,33 +970,182 @@ static int grid_sort_into_a(bs_engine* e)
     return BS_OK;
 }
 
-static int upload_f64(bs_engine* e, const double* pos3, const double* vel3)
-{
-    const uint32_t n = e->prm.n;
-    std::vector<double> buf(7 * (size_t)n);
-    double *x = buf.data(), *y = x + n, *z = y + n, *vx = z + n, *vy = vx + n, *vz = vy + n;
-    uint32_t* ids = (uint32_t*)(vz + n);
-    for (uint32_t i = 0; i < n; ++i) {
-        x[i] = pos3[3 * (size_t)i]; y[i] = pos3[3 * (size_t)i + 1]; z[i] = pos3[3 * (size_t)i + 2];
-        vx[i] = vel3[3 * (size_t)i]; vy[i] = vel3[3 * (size_t)i + 1]; vz[i] = vel3[3 * (size_t)i + 2];
-        ids[i] = i;
+// How states and forces go in and out (24 bytes a boid in, 48 out; "before" is
+// the runtime's copy from or to the caller's pageable memory, one per array):
+//   up to kDirect: through the staging in parts, one part copied on the host
+//     while the next is under way (in: 10^4 boids 137 -> 60 us, 130000 boids 608
+//     -> 190 us; out, after queued updates: 14000 boids 101 -> 82 us, 130000
+//     402 -> 252 us);
+//   above it: in pieces of kPiece that up to kStageThreads threads carry, each
+//     through a piece of the staging of its own, so the copies to and from
+//     the caller's pages (a few GB/s a thread, page faults included) run
+//     beside one another and the DMA (2^20 boids: in 17.5 -> 1.0 ms, out 5.4
+//     -> 1.6 ms; below it starting the threads costs more than they save:
+//     130000 boids out 289 us).
+constexpr size_t kPiece = (size_t)2 << 20, kPart = (size_t)1 << 18, kDirect = (size_t)8 << 20;
+constexpr unsigned kStageThreads = 6;
+// States up to this size are written to the staging by the kernel that puts
+// them in order (consecutive words), without a copy after it.
+constexpr size_t kMapped = (size_t)1 << 19;
+static_assert(kStageThreads <= sizeof(((bs_engine*)0)->stage_ev) / sizeof(hipEvent_t), "an event per thread");
+
+// A call's hold on the staging it uses; `reader` is a stream that may still
+// be copying out of it when the call ends.
+struct StageLoan {
+    char* p = nullptr;
+    size_t bytes = 0;
+    hipStream_t reader = nullptr;
+    ~StageLoan()
+    {
+        if (reader) (void)hipStreamSynchronize(reader);
+        stage_back(p, bytes);
     }
-    const bool grid = is_grid(e->mode);
-    StateF64 dst = grid ? e->db : e->da;
-    const size_t b = sizeof(double) * n;
-    HIP_TRY(e, hipMemcpyAsync(dst.x, x, b, hipMemcpyHostToDevice, e->stream));
-    HIP_TRY(e, hipMemcpyAsync(dst.y, y, b, hipMemcpyHostToDevice, e->stream));
-    HIP_TRY(e, hipMemcpyAsync(dst.z, z, b, hipMemcpyHostToDevice, e->stream));
-    HIP_TRY(e, hipMemcpyAsync(dst.vx, vx, b, hipMemcpyHostToDevice, e->stream));
-    HIP_TRY(e, hipMemcpyAsync(dst.vy, vy, b, hipMemcpyHostToDevice, e->stream));
-    HIP_TRY(e, hipMemcpyAsync(dst.vz, vz, b, hipMemcpyHostToDevice, e->stream));
-    HIP_TRY(e, hipMemcpyAsync(dst.id, ids, sizeof(uint32_t) * n, hipMemcpyHostToDevice, e->stream));
-    if (grid) {
-        HIP_TRY(e, launch_hash_count(flock_view(e), e->db, e->key, e->rank, e->count, e->stream));
+};
+
+// Staging of at least `bytes` (at most kStageThreads pieces) for this call;
+// false where there is none (the caller then copies from and to pageable
+// memory).
+static bool lend_stage(bs_engine* e, size_t bytes, StageLoan& loan)
+{
+    const size_t want = std::min(bytes, kStageThreads * kPiece);
+    for (auto& ev : e->stage_ev)
+        if (!ev && hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
+            ev = nullptr;
+            (void)hipGetLastError();
+            return false;
+        }
+    loan.p = stage_take(want, &loan.bytes);
+    return loan.p != nullptr;
+}
+
+// Up to two host arrays and the device buffer that holds them end to end.
+struct Span { char* host; size_t bytes; };
+
+#ifndef MADV_POPULATE_WRITE
+#define MADV_POPULATE_WRITE 23
+#endif
+// Maps the pages of [p, p + bytes) for writing, where the kernel can do so in
+// one call (Linux 5.14; else they fault in one by one later).  The contents
+// stay as they are.  A result array is mostly fresh memory, and taken here its
+// page faults (0.4 us each) pass while the device finishes the updates queued
+// before (50021 boids: 157 us after the updates, 470 us without).
+static void prefault(char* p, size_t bytes)
+{
+    const uintptr_t page = 4096, lo = ((uintptr_t)p + page - 1) & ~(page - 1), hi = ((uintptr_t)p + bytes) & ~(page - 1);
+    if (hi > lo + 4 * page) (void)madvise((void*)lo, hi - lo, MADV_POPULATE_WRITE);
+}
+
+static void copy_part(const Span* a, size_t at, char* stage, size_t bytes, bool to_host)
+{
+    size_t first = 0;
+    for (int k = 0; k < 2 && bytes; ++k) {
+        const size_t end = first + a[k].bytes;
+        if (at < end && a[k].bytes) {
+            const size_t off = at - first, len = std::min(bytes, a[k].bytes - off);
+            if (to_host) memcpy(a[k].host + off, stage, len); else memcpy(stage, a[k].host + off, len);
+            stage += len; at += len; bytes -= len;
+        }
+        first = end;
+    }
+}
+
+// Copies the two arrays (end to end at dev) to or from the device, after the
+// work queued on the engine's stream; returns once done, except that a copy to
+// the device may still be reading the staging (loan.reader).
+static int transfer(bs_engine* e, const Span (&a)[2], char* dev, bool to_host, StageLoan& loan)
+{
+    const size_t total = a[0].bytes + a[1].bytes;
+    if (total == 0) { HIP_TRY(e, hipStreamSynchronize(e->stream)); return BS_OK; }
+    const bool direct = total <= kDirect;
+    if (!lend_stage(e, total, loan)) {
+        size_t at = 0;
+        for (const Span& s : a) {
+            if (s.bytes)
+                HIP_TRY(e, to_host ? hipMemcpyAsync(s.host, dev + at, s.bytes, hipMemcpyDeviceToHost, e->stream)
+                                   : hipMemcpyAsync(dev + at, s.host, s.bytes, hipMemcpyHostToDevice, e->stream));
+            at += s.bytes;
+        }
+        HIP_TRY(e, hipStreamSynchronize(e->stream));
+        return BS_OK;
+    }
+    if (direct && to_host) {
+        // in parts: one leaves the staging while the next arrives
+        const size_t part = total <= 2 * kPart ? total : std::max(kPart, (total / kStageThreads + 4095) & ~(size_t)4095);
+        const unsigned parts = (unsigned)((total + part - 1) / part);
+        for (unsigned k = 0; k < parts; ++k) {
+            const size_t at = k * part, len = std::min(part, total - at);
+            HIP_TRY(e, hipMemcpyAsync(loan.p + at, dev + at, len, hipMemcpyDeviceToHost, e->stream));
+            if (k + 1 < parts) HIP_TRY(e, hipEventRecord(e->stage_ev[k], e->stream));
+        }
+        for (const Span& s : a) prefault(s.host, s.bytes);
+        for (unsigned k = 0; k < parts; ++k) {
+            const size_t at = k * part;
+            HIP_TRY(e, k + 1 < parts ? hipEventSynchronize(e->stage_ev[k]) : hipStreamSynchronize(e->stream));
+            copy_part(a, at, loan.p + at, std::min(part, total - at), true);
+        }
+        return BS_OK;
+    }
+    if (direct) {
+        loan.reader = e->stream;
+        for (size_t at = 0; at < total; at += kPart) {
+            const size_t len = std::min(kPart, total - at);
+            copy_part(a, at, loan.p + at, len, false);
+            HIP_TRY(e, hipMemcpyAsync(dev + at, loan.p + at, len, hipMemcpyHostToDevice, e->stream));
+        }
+        return BS_OK;
+    }
+    const size_t pieces = (total + kPiece - 1) / kPiece;
+    const unsigned cpus = std::max(1u, std::thread::hardware_concurrency());
+    const unsigned threads = (unsigned)std::min<size_t>(std::min<size_t>(pieces, loan.bytes / kPiece),
+                                                        std::min(kStageThreads, cpus));
+    std::atomic<size_t> next{0};
+    std::atomic<int> error{(int)hipSuccess};
+    auto carry = [&](unsigned w) {
+        char* stage = loan.p + w * kPiece;
+        hipError_t st = hipSetDevice(e->device);
+        if (to_host)                                         // its share of the caller's pages
+            for (const Span& s : a) {
+                const size_t share = (s.bytes / threads + 4095) & ~(size_t)4095, from = std::min(s.bytes, w * share);
+                prefault(s.host + from, std::min(share, s.bytes - from));
+            }
+        for (size_t k; st == hipSuccess && error.load() == (int)hipSuccess && (k = next.fetch_add(1)) < pieces;) {
+            const size_t at = k * kPiece, len = std::min(kPiece, total - at);
+            if (!to_host) copy_part(a, at, stage, len, false);
+            st = to_host ? hipMemcpyAsync(stage, dev + at, len, hipMemcpyDeviceToHost, e->stream)
+                         : hipMemcpyAsync(dev + at, stage, len, hipMemcpyHostToDevice, e->stream);
+            if (st == hipSuccess) st = hipEventRecord(e->stage_ev[w], e->stream);
+            if (st == hipSuccess) st = hipEventSynchronize(e->stage_ev[w]);
+            if (st == hipSuccess && to_host) copy_part(a, at, stage, len, true);
+        }
+        if (st != hipSuccess) error.store((int)st);
+    };
+    std::thread helpers[kStageThreads];
+    unsigned started = 0;
+    for (unsigned w = 1; w < threads; ++w) {
+        try {
+            helpers[started] = std::thread(carry, w);
+            ++started;
+        } catch (const std::system_error&) {
+            break;                                           // no more threads: the started ones carry it all
+        }
+    }
+    carry(0);
+    for (unsigned w = 0; w < started; ++w) helpers[w].join();
+    HIP_TRY(e, (hipError_t)error.load());
+    return BS_OK;
+}
+
+// The state uploaded to the device (st, id order), sorted where the engine
+// keeps it sorted; returns once done.
+static int settle_state(bs_engine* e, StateF64 st, StageLoan& loan)
+{
+    if (is_grid(e->mode)) {
+        HIP_TRY(e, launch_hash_count(flock_view(e), st, e->key, e->rank, e->count, e->stream));
         int rc = grid_sort_into_a(e);
         if (rc) return rc;
     }
-    HIP_TRY(e, hipStreamSynchronize(e->stream));   // the host staging buffer dies here
+    HIP_TRY(e, hipStreamSynchronize(e->stream));
+    loan.reader = nullptr;
     e->has_state = true;
     e->steps = 0;
     return BS_OK;
@@ -922,9 +1154,16 @@ static int upload_f64(bs_engine* e, const double* pos3, const double* vel3)
 extern "C" int bs_set_state_f64(bs_engine* e, const double* pos3, const double* vel3)
 {
     if (!e) return BS_E_ARG;
-    if (e->prm.n && (!pos3 || !vel3)) return fail(e, BS_E_ARG, "bs_set_state_f64: NULL array");
+    const uint32_t n = e->prm.n;
+    if (n && (!pos3 || !vel3)) return fail(e, BS_E_ARG, "bs_set_state_f64: NULL array");
     if (is_f32(e->mode)) return fail(e, BS_E_STATE, "float-state mode: use bs_set_state_f32");
-    return upload_f64(e, pos3, vel3);
+    const StateF64 st = is_grid(e->mode) ? e->db : e->da;
+    const Span a[2] = {{(char*)pos3, sizeof(double) * 3 * n}, {(char*)vel3, sizeof(double) * 3 * n}};
+    StageLoan loan;
+    int rc = transfer(e, a, (char*)e->tmp_pos, false, loan);
+    if (rc) return rc;
+    HIP_TRY(e, launch_unpack(n, e->tmp_pos, e->tmp_vel, st, e->stream));
+    return settle_state(e, st, loan);
 }
 
 extern "C" int bs_set_state_f32(bs_engine* e, const float* xyzv6)
@@ -932,25 +1171,21 @@ extern "C" int bs_set_state_f32(bs_engine* e, const float* xyzv6)
     if (!e) return BS_E_ARG;
     const uint32_t n = e->prm.n;
     if (n && !xyzv6) return fail(e, BS_E_ARG, "bs_set_state_f32: NULL array");
+    const Span a[2] = {{(char*)xyzv6, sizeof(float) * 6 * n}, {nullptr, 0}};
+    StageLoan loan;
+    int rc = transfer(e, a, (char*)e->tmp_pos, false, loan);
+    if (rc) return rc;
     if (is_f32(e->mode)) {
-        std::vector<float> buf(6 * (size_t)n);
-        for (uint32_t i = 0; i < n; ++i)
-            for (int k = 0; k < 6; ++k) buf[(size_t)k * n + i] = xyzv6[6 * (size_t)i + k];
-        float* dst[6] = {e->fa.x, e->fa.y, e->fa.z, e->fa.vx, e->fa.vy, e->fa.vz};
-        for (int k = 0; k < 6; ++k)
-            HIP_TRY(e, hipMemcpyAsync(dst[k], buf.data() + (size_t)k * n, sizeof(float) * n, hipMemcpyHostToDevice, e->stream));
+        HIP_TRY(e, launch_unpack(n, (const float*)e->tmp_pos, e->fa, e->stream));
         HIP_TRY(e, hipStreamSynchronize(e->stream));
+        loan.reader = nullptr;
         e->has_state = true;
         e->steps = 0;
         return BS_OK;
     }
-    std::vector<double> pos(3 * (size_t)n), vel(3 * (size_t)n);
-    for (uint32_t i = 0; i < n; ++i)
-        for (int k = 0; k < 3; ++k) {
-            pos[3 * (size_t)i + k] = xyzv6[6 * (size_t)i + k];
-            vel[3 * (size_t)i + k] = xyzv6[6 * (size_t)i + 3 + k];
-        }
-    return upload_f64(e, pos.data(), vel.data());
+    const StateF64 st = is_grid(e->mode) ? e->db : e->da;
+    HIP_TRY(e, launch_unpack(n, (const float*)e->tmp_pos, st, e->stream));
+    return settle_state(e, st, loan);
 }
 
 // Reports a chunk table cut short by its capacity (k_rows_pass clamps the
@@ -960,94 +1195,89 @@ extern "C" int bs_set_state_f32(bs_engine* e, const float* xyzv6)
 static int check_grid(bs_engine* e)
 {
     if (!e->overflow) return BS_OK;
-    uint32_t v = 0;
-    HIP_TRY(e, hipMemcpyAsync(&v, e->overflow, sizeof(uint32_t), hipMemcpyDeviceToHost, e->stream));
     HIP_TRY(e, hipStreamSynchronize(e->stream));
+    const uint32_t v = *(volatile uint32_t*)e->overflow;
     if (v)
         return fail(e, BS_E_STATE, "chunk table overflow: " + std::to_string(v) + " chunks for a capacity of " +
                                        std::to_string(e->max_chunks) + " (results invalid)");
     return BS_OK;
 }
 
-extern "C" int bs_get_state_f64(bs_engine* e, double* pos3, double* vel3)
+// The state in id order as T, out through tmp_pos.
+template <typename T>
+static int get_state(bs_engine* e, T* pos3, T* vel3, const char* what)
 {
     if (!e) return BS_E_ARG;
     const uint32_t n = e->prm.n;
-    if (n && (!pos3 || !vel3)) return fail(e, BS_E_ARG, "bs_get_state_f64: NULL array");
+    if (n && (!pos3 || !vel3)) return fail(e, BS_E_ARG, std::string(what) + ": NULL array");
     if (!e->has_state) return fail(e, BS_E_STATE, "no state: call bs_set_state_* first");
-    if (is_f32(e->mode)) {
-        std::vector<float> p(3 * (size_t)n), v(3 * (size_t)n);
-        int rc = bs_get_state_f32(e, p.data(), v.data());
-        if (rc) return rc;
-        for (size_t k = 0; k < 3 * (size_t)n; ++k) { pos3[k] = p[k]; vel3[k] = v[k]; }
-        return BS_OK;
+    T* tmp = (T*)e->tmp_pos;
+    const size_t bytes = sizeof(T) * 6 * n;
+    StageLoan loan;
+    if (bytes <= kMapped && !is_grid(e->mode) && lend_stage(e, bytes, loan)) {
+        // small states in id order: the kernel writes the staging itself
+        T* out = (T*)loan.p;
+        if (is_f32(e->mode)) HIP_TRY(e, launch_pack_f32(n, e->fa, out, out + 3 * (size_t)n, e->stream));
+        else HIP_TRY(e, launch_pack_f64(n, e->da, out, out + 3 * (size_t)n, e->stream));
+        prefault((char*)pos3, bytes / 2);
+        prefault((char*)vel3, bytes / 2);
+        HIP_TRY(e, hipStreamSynchronize(e->stream));
+        memcpy(pos3, out, bytes / 2);
+        memcpy(vel3, out + 3 * (size_t)n, bytes / 2);
+        return check_grid(e);
     }
-    HIP_TRY(e, launch_unsort_f64(n, e->da, e->tmp_pos, e->tmp_vel, e->stream));
-    HIP_TRY(e, hipMemcpyAsync(pos3, e->tmp_pos, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, e->stream));
-    HIP_TRY(e, hipMemcpyAsync(vel3, e->tmp_vel, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, e->stream));
-    HIP_TRY(e, hipStreamSynchronize(e->stream));
-    return check_grid(e);
+    if (is_f32(e->mode)) HIP_TRY(e, launch_pack_f32(n, e->fa, tmp, tmp + 3 * (size_t)n, e->stream));
+    else HIP_TRY(e, launch_unsort_f64(n, e->da, tmp, tmp + 3 * (size_t)n, e->stream));
+    const Span a[2] = {{(char*)pos3, sizeof(T) * 3 * n}, {(char*)vel3, sizeof(T) * 3 * n}};
+    int rc = transfer(e, a, (char*)tmp, true, loan);
+    return rc ? rc : check_grid(e);
+}
+
+extern "C" int bs_get_state_f64(bs_engine* e, double* pos3, double* vel3)
+{
+    return get_state(e, pos3, vel3, "bs_get_state_f64");
 }
 
 extern "C" int bs_get_state_f32(bs_engine* e, float* pos3, float* vel3)
 {
-    if (!e) return BS_E_ARG;
-    const uint32_t n = e->prm.n;
-    if (n && (!pos3 || !vel3)) return fail(e, BS_E_ARG, "bs_get_state_f32: NULL array");
-    if (!e->has_state) return fail(e, BS_E_STATE, "no state: call bs_set_state_* first");
-    if (is_f32(e->mode)) {
-        std::vector<float> buf(6 * (size_t)n);
-        float* src[6] = {e->fa.x, e->fa.y, e->fa.z, e->fa.vx, e->fa.vy, e->fa.vz};
-        for (int k = 0; k < 6; ++k)
-            HIP_TRY(e, hipMemcpyAsync(buf.data() + (size_t)k * n, src[k], sizeof(float) * n, hipMemcpyDeviceToHost, e->stream));
-        HIP_TRY(e, hipStreamSynchronize(e->stream));
-        for (uint32_t i = 0; i < n; ++i)
-            for (int k = 0; k < 3; ++k) {
-                pos3[3 * (size_t)i + k] = buf[(size_t)k * n + i];
-                vel3[3 * (size_t)i + k] = buf[(size_t)(3 + k) * n + i];
-            }
-        return BS_OK;
-    }
-    std::vector<double> p(3 * (size_t)n), v(3 * (size_t)n);
-    int rc = bs_get_state_f64(e, p.data(), v.data());
-    if (rc) return rc;
-    for (size_t k = 0; k < 3 * (size_t)n; ++k) { pos3[k] = (float)p[k]; vel3[k] = (float)v[k]; }
-    return BS_OK;
+    return get_state(e, pos3, vel3, "bs_get_state_f32");
 }
 
 extern "C" int bs_get_forces_f64(bs_engine* e, double* f9)
 {
     if (!e) return BS_E_ARG;
-    const uint32_t n = e->prm.n;
+    const size_t n9 = 9 * (size_t)e->prm.n;
     if (!e->forces) return fail(e, BS_E_STATE, "engine created without BS_FLAG_FORCES");
-    if (n && !f9) return fail(e, BS_E_ARG, "bs_get_forces_f64: NULL array");
+    if (n9 && !f9) return fail(e, BS_E_ARG, "bs_get_forces_f64: NULL array");
     if (is_f32(e->mode)) {
-        std::vector<float> tmp(9 * (size_t)n);
-        HIP_TRY(e, hipMemcpyAsync(tmp.data(), e->forces, sizeof(float) * 9 * n, hipMemcpyDeviceToHost, e->stream));
-        HIP_TRY(e, hipStreamSynchronize(e->stream));
-        for (size_t k = 0; k < tmp.size(); ++k) f9[k] = tmp[k];
+        std::vector<float> tmp(n9);
+        const Span a[2] = {{(char*)tmp.data(), sizeof(float) * n9}, {nullptr, 0}};
+        StageLoan loan;
+        int rc = transfer(e, a, (char*)e->forces, true, loan);
+        if (rc) return rc;
+        for (size_t k = 0; k < n9; ++k) f9[k] = tmp[k];
         return BS_OK;
     }
-    HIP_TRY(e, hipMemcpyAsync(f9, e->forces, sizeof(double) * 9 * n, hipMemcpyDeviceToHost, e->stream));
-    HIP_TRY(e, hipStreamSynchronize(e->stream));
-    return BS_OK;
+    const Span a[2] = {{(char*)f9, sizeof(double) * n9}, {nullptr, 0}};
+    StageLoan loan;
+    return transfer(e, a, (char*)e->forces, true, loan);
 }
 
 extern "C" int bs_get_forces_f32(bs_engine* e, float* f9)
 {
     if (!e) return BS_E_ARG;
-    const uint32_t n = e->prm.n;
+    const size_t n9 = 9 * (size_t)e->prm.n;
     if (!e->forces) return fail(e, BS_E_STATE, "engine created without BS_FLAG_FORCES");
-    if (n && !f9) return fail(e, BS_E_ARG, "bs_get_forces_f32: NULL array");
+    if (n9 && !f9) return fail(e, BS_E_ARG, "bs_get_forces_f32: NULL array");
     if (is_f32(e->mode)) {
-        HIP_TRY(e, hipMemcpyAsync(f9, e->forces, sizeof(float) * 9 * n, hipMemcpyDeviceToHost, e->stream));
-        HIP_TRY(e, hipStreamSynchronize(e->stream));
-        return BS_OK;
+        const Span a[2] = {{(char*)f9, sizeof(float) * n9}, {nullptr, 0}};
+        StageLoan loan;
+        return transfer(e, a, (char*)e->forces, true, loan);
     }
-    std::vector<double> tmp(9 * (size_t)n);
+    std::vector<double> tmp(n9);
     int rc = bs_get_forces_f64(e, tmp.data());
     if (rc) return rc;
-    for (size_t k = 0; k < tmp.size(); ++k) f9[k] = (float)tmp[k];
+    for (size_t k = 0; k < n9; ++k) f9[k] = (float)tmp[k];
     return BS_OK;
 }
 
@@ -1078,8 +1308,8 @@ extern "C" int bs_debug_grid(bs_engine* e, uint32_t* key_sorted, uint32_t* id_so
     info->chunk_boids = (int32_t)e->chunk;
     info->chunk_span = e->cspan;
     HIP_TRY(e, hipMemcpyAsync(&info->nchunks, e->nchunks, sizeof(uint32_t), hipMemcpyDeviceToHost, e->stream));
-    HIP_TRY(e, hipMemcpyAsync(&info->overflow, e->overflow, sizeof(uint32_t), hipMemcpyDeviceToHost, e->stream));
     HIP_TRY(e, hipStreamSynchronize(e->stream));
+    info->overflow = *(volatile uint32_t*)e->overflow;
     if (key_sorted)
         HIP_TRY(e, hipMemcpyAsync(key_sorted, e->key_sorted, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, e->stream));
     if (id_sorted)
@@ -1328,7 +1558,7 @@ static int metrics_impl(bs_engine* e, uint32_t flock, double eps, uint32_t min_s
                                      std::to_string(kScratchBytes) + " bytes): use bs_metrics_flock");
     if (static_ws && !e->scratch) return fail(e, BS_E_STATE, "static scratch unavailable: " + e->scratch_why);
     if (is_f32(e->mode))
-        HIP_TRY(e, launch_f32_to_f64(ntot, e->fa, e->tmp_pos, e->tmp_vel, e->stream));
+        HIP_TRY(e, launch_pack_f32(ntot, e->fa, e->tmp_pos, e->tmp_vel, e->stream));
     else
         HIP_TRY(e, launch_unsort_f64(ntot, e->da, e->tmp_pos, e->tmp_vel, e->stream));
     void* ws = nullptr;

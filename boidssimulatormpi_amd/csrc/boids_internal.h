@@ -169,8 +169,17 @@ size_t metrics_priced_bytes(uint32_t n, int G);
 hipError_t launch_metrics(uint32_t n, double F, int G, double eps, uint32_t min_size, const double* pos3,
                           const double* vel3, void* ws, size_t ws_bytes, double** out4_dev,
                           hipStream_t stream);
-hipError_t launch_f32_to_f64(uint32_t n, StateF32 st, double* pos3, double* vel3, hipStream_t stream);
-hipError_t launch_unsort_f64(uint32_t n, StateF64 src, double* pos3, double* vel3,
-                             hipStream_t stream);
+// State out (id order, n x 3 each) and in (n x 3 each, or n x 6 interleaved).
+// n <= 2^28, so 3 n fits 32 bits.
+hipError_t launch_unsort_f64(uint32_t n, StateF64 src, double* pos3, double* vel3, hipStream_t stream);
+hipError_t launch_unsort_f64(uint32_t n, StateF64 src, float* pos3, float* vel3, hipStream_t stream);
+hipError_t launch_pack_f32(uint32_t n, StateF32 st, float* pos3, float* vel3, hipStream_t stream);
+hipError_t launch_pack_f32(uint32_t n, StateF32 st, double* pos3, double* vel3, hipStream_t stream);
+// (the FP64 all-pairs state, in id order itself)
+hipError_t launch_pack_f64(uint32_t n, StateF64 st, float* pos3, float* vel3, hipStream_t stream);
+hipError_t launch_pack_f64(uint32_t n, StateF64 st, double* pos3, double* vel3, hipStream_t stream);
+hipError_t launch_unpack(uint32_t n, const double* pos3, const double* vel3, StateF64 st, hipStream_t stream);
+hipError_t launch_unpack(uint32_t n, const float* xyzv6, StateF64 st, hipStream_t stream);
+hipError_t launch_unpack(uint32_t n, const float* xyzv6, StateF32 st, hipStream_t stream);
 
 }  // namespace boids

@@ -400,14 +400,49 @@ __global__ __launch_bounds__(kBlock) void k_gather(Flocks F, const uint32_t* per
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_unsort_f64(uint32_t n, StateF64 src, double* pos3,
-                                                       double* vel3)
+// State in id order, three values per boid (T = the type the caller asked for).
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_unsort_f64(uint32_t n, StateF64 src, T* pos3, T* vel3)
 {
     const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
     if (s >= n) return;
     const size_t i = src.id[s];
-    pos3[3 * i] = src.x[s]; pos3[3 * i + 1] = src.y[s]; pos3[3 * i + 2] = src.z[s];
-    vel3[3 * i] = src.vx[s]; vel3[3 * i + 1] = src.vy[s]; vel3[3 * i + 2] = src.vz[s];
+    pos3[3 * i] = (T)src.x[s]; pos3[3 * i + 1] = (T)src.y[s]; pos3[3 * i + 2] = (T)src.z[s];
+    vel3[3 * i] = (T)src.vx[s]; vel3[3 * i + 1] = (T)src.vy[s]; vel3[3 * i + 2] = (T)src.vz[s];
+}
+
+// A state that is in id order already, one value per thread: consecutive
+// threads write consecutive words, also where out lies in host memory.
+template <typename T, typename St>
+__global__ __launch_bounds__(kBlock) void k_pack(uint32_t n, St st, T* pos3, T* vel3)
+{
+    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+    const uint32_t i = k / 3, c = k - 3 * i;
+    if (i >= n) return;
+    pos3[k] = (T)(c == 0 ? st.x : c == 1 ? st.y : st.z)[i];
+    vel3[k] = (T)(c == 0 ? st.vx : c == 1 ? st.vy : st.vz)[i];
+}
+
+// Uploaded state: pos and vel hold boid i's three values at stride * i.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_unpack_f64(uint32_t n, const T* __restrict__ pos,
+                                                       const T* __restrict__ vel, uint32_t stride, StateF64 st)
+{
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    const T *p = pos + (size_t)stride * i, *v = vel + (size_t)stride * i;
+    st.x[i] = p[0]; st.y[i] = p[1]; st.z[i] = p[2];
+    st.vx[i] = v[0]; st.vy[i] = v[1]; st.vz[i] = v[2];
+    st.id[i] = i;
+}
+
+__global__ __launch_bounds__(kBlock) void k_unpack_f32(uint32_t n, const float* __restrict__ xyzv6, StateF32 st)
+{
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    const float* p = xyzv6 + 6 * (size_t)i;
+    st.x[i] = p[0]; st.y[i] = p[1]; st.z[i] = p[2];
+    st.vx[i] = p[3]; st.vy[i] = p[4]; st.vz[i] = p[5];
 }
 
 // Launchers
@@ -524,11 +559,66 @@ hipError_t launch_copy(const void* src, void* dst, uint64_t bytes, hipStream_t s
     return hipGetLastError();
 }
 
-hipError_t launch_unsort_f64(uint32_t n, StateF64 src, double* pos3, double* vel3,
-                             hipStream_t stream)
+hipError_t launch_unsort_f64(uint32_t n, StateF64 src, double* pos3, double* vel3, hipStream_t stream)
 {
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_unsort_f64, dim3(blocks_for(n)), dim3(kBlock), 0, stream, n, src, pos3, vel3);
+    hipLaunchKernelGGL(k_unsort_f64<double>, dim3(blocks_for(n)), dim3(kBlock), 0, stream, n, src, pos3, vel3);
+    return hipGetLastError();
+}
+
+hipError_t launch_unsort_f64(uint32_t n, StateF64 src, float* pos3, float* vel3, hipStream_t stream)
+{
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_unsort_f64<float>, dim3(blocks_for(n)), dim3(kBlock), 0, stream, n, src, pos3, vel3);
+    return hipGetLastError();
+}
+
+hipError_t launch_pack_f32(uint32_t n, StateF32 st, float* pos3, float* vel3, hipStream_t stream)
+{
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL((k_pack<float, StateF32>), dim3(blocks_for(3 * n)), dim3(kBlock), 0, stream, n, st, pos3, vel3);
+    return hipGetLastError();
+}
+
+hipError_t launch_pack_f32(uint32_t n, StateF32 st, double* pos3, double* vel3, hipStream_t stream)
+{
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL((k_pack<double, StateF32>), dim3(blocks_for(3 * n)), dim3(kBlock), 0, stream, n, st, pos3, vel3);
+    return hipGetLastError();
+}
+
+hipError_t launch_pack_f64(uint32_t n, StateF64 st, float* pos3, float* vel3, hipStream_t stream)
+{
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL((k_pack<float, StateF64>), dim3(blocks_for(3 * n)), dim3(kBlock), 0, stream, n, st, pos3, vel3);
+    return hipGetLastError();
+}
+
+hipError_t launch_pack_f64(uint32_t n, StateF64 st, double* pos3, double* vel3, hipStream_t stream)
+{
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL((k_pack<double, StateF64>), dim3(blocks_for(3 * n)), dim3(kBlock), 0, stream, n, st, pos3, vel3);
+    return hipGetLastError();
+}
+
+hipError_t launch_unpack(uint32_t n, const double* pos3, const double* vel3, StateF64 st, hipStream_t stream)
+{
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_unpack_f64<double>, dim3(blocks_for(n)), dim3(kBlock), 0, stream, n, pos3, vel3, 3u, st);
+    return hipGetLastError();
+}
+
+hipError_t launch_unpack(uint32_t n, const float* xyzv6, StateF64 st, hipStream_t stream)
+{
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_unpack_f64<float>, dim3(blocks_for(n)), dim3(kBlock), 0, stream, n, xyzv6, xyzv6 + 3, 6u, st);
+    return hipGetLastError();
+}
+
+hipError_t launch_unpack(uint32_t n, const float* xyzv6, StateF32 st, hipStream_t stream)
+{
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_unpack_f32, dim3(blocks_for(n)), dim3(kBlock), 0, stream, n, xyzv6, st);
     return hipGetLastError();
 }
 

@@ -73,15 +73,6 @@ __global__ __launch_bounds__(kBlock) void k_m_order(MGrid g, const double* pos3,
 
 __device__ __forceinline__ uint32_t m_id(const double4& q) { return (uint32_t)__double_as_longlong(q.w); }
 
-// float SoA state (reference-faithful mode) -> double AoS
-__global__ __launch_bounds__(kBlock) void k_m_from_f32(uint32_t n, StateF32 st, double* pos3, double* vel3)
-{
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    pos3[3 * (size_t)i] = st.x[i]; pos3[3 * (size_t)i + 1] = st.y[i]; pos3[3 * (size_t)i + 2] = st.z[i];
-    vel3[3 * (size_t)i] = st.vx[i]; vel3[3 * (size_t)i + 1] = st.vy[i]; vel3[3 * (size_t)i + 2] = st.vz[i];
-}
-
 __global__ __launch_bounds__(kBlock) void k_m_fill(uint32_t* a, uint32_t n, uint32_t v)
 {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
@@ -327,13 +318,6 @@ __global__ __launch_bounds__(kBlock) void k_m_results(uint32_t n, uint32_t block
 }
 
 static inline uint32_t mblocks(uint32_t n) { return (n + kBlock - 1) / kBlock; }
-
-hipError_t launch_f32_to_f64(uint32_t n, StateF32 st, double* pos3, double* vel3, hipStream_t stream)
-{
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_m_from_f32, dim3(mblocks(n)), dim3(kBlock), 0, stream, n, st, pos3, vel3);
-    return hipGetLastError();
-}
 
 // Workspace layout: one function carves the regions, both for sizing
 // (base == nullptr) and for the launch, so the two cannot disagree.

@@ -246,26 +246,26 @@ class Engine:
         self._check(lib().bs_sync(self._h), "bs_sync")
 
     def state_f64(self):
-        p = np.zeros((self.n, 3), np.float64)
-        v = np.zeros((self.n, 3), np.float64)
+        p = np.empty((self.n, 3), np.float64)
+        v = np.empty((self.n, 3), np.float64)
         self._check(lib().bs_get_state_f64(self._h, _p(p, ctypes.c_double), _p(v, ctypes.c_double)),
                     "bs_get_state_f64")
         return p, v
 
     def state_f32(self):
-        p = np.zeros((self.n, 3), np.float32)
-        v = np.zeros((self.n, 3), np.float32)
+        p = np.empty((self.n, 3), np.float32)
+        v = np.empty((self.n, 3), np.float32)
         self._check(lib().bs_get_state_f32(self._h, _p(p, ctypes.c_float), _p(v, ctypes.c_float)),
                     "bs_get_state_f32")
         return p, v
 
     def forces_f64(self):
-        f = np.zeros((self.n, 9), np.float64)
+        f = np.empty((self.n, 9), np.float64)
         self._check(lib().bs_get_forces_f64(self._h, _p(f, ctypes.c_double)), "bs_get_forces_f64")
         return f
 
     def forces_f32(self):
-        f = np.zeros((self.n, 9), np.float32)
+        f = np.empty((self.n, 9), np.float32)
         self._check(lib().bs_get_forces_f32(self._h, _p(f, ctypes.c_float)), "bs_get_forces_f32")
         return f
 
