@@ -202,7 +202,7 @@ struct bs_engine {
     bool capturing = false;
     Lattice lat{};
     double2* rec = nullptr;            // FP64 grid: interleaved pair records
-    float4 *rec4 = nullptr, *vrec4 = nullptr;   // float grid: sorted positions (+ id) and velocities
+    float4* rec4 = nullptr;            // float grid: positions and ids by cell
     uint32_t* recheck = nullptr;
     uint32_t* overflow = nullptr;      // chunk-table count beyond its capacity (0: none), in pinned host memory
     void* scratch = nullptr;           // this device's static scratch (allocation-free entry points)
@@ -823,10 +823,9 @@ static int create_engine(const bs_params* fp, uint32_t count, bool batch, bs_eng
     if (p->flags & BS_FLAG_DIGEST) { if ((rc = dev_alloc(e, &e->digest, 4 * (size_t)n))) return bail(rc); }
     if (e->mode == BS_MODE_GRID_F32REF) {
         const uint32_t ntiles = (e->ncell1 + 4095) / 4096;
-        if ((rc = dev_alloc(e, &e->key, n)) || (rc = dev_alloc(e, &e->rank, n)) || (rc = dev_alloc(e, &e->perm, n)) ||
+        if ((rc = dev_alloc(e, &e->key, n)) || (rc = dev_alloc(e, &e->rank, n)) ||
             (rc = dev_alloc(e, &e->count, e->ncell1)) || (rc = dev_alloc(e, &e->start, e->ncell1)) ||
-            (rc = dev_alloc(e, &e->partials, ntiles)) || (rc = dev_alloc(e, &e->rec4, n)) ||
-            (rc = dev_alloc(e, &e->vrec4, n)))
+            (rc = dev_alloc(e, &e->partials, ntiles)) || (rc = dev_alloc(e, &e->rec4, n)))
             return bail(rc);
         st = hipMemsetAsync(e->count, 0, sizeof(uint32_t) * e->ncell1, e->stream);
         if (st != hipSuccess) { hip_fail(e, st, "hipMemsetAsync"); return bail(BS_E_HIP); }
@@ -1177,6 +1176,10 @@ extern "C" int bs_set_state_f32(bs_engine* e, const float* xyzv6)
     if (rc) return rc;
     if (is_f32(e->mode)) {
         HIP_TRY(e, launch_unpack(n, (const float*)e->tmp_pos, e->fa, e->stream));
+        if (e->mode == BS_MODE_GRID_F32REF) {                // the last state's counts give way to this one's
+            HIP_TRY(e, hipMemsetAsync(e->count, 0, sizeof(uint32_t) * e->ncell1, e->stream));
+            HIP_TRY(e, launch_f32_hash(e->P, e->fa, e->key, e->rank, e->count, e->stream));
+        }
         HIP_TRY(e, hipStreamSynchronize(e->stream));
         loan.reader = nullptr;
         e->has_state = true;
@@ -1390,11 +1393,11 @@ extern "C" int bs_step(bs_engine* e, uint32_t nsteps)
         }
         case BS_MODE_GRID_F32REF: {
             Timed ts(e, BS_K_SCAN);
-            HIP_TRY(e, launch_f32_grid_sort(e->P, e->fa, e->key, e->rank, e->count, e->start, e->partials, e->perm,
-                                            e->rec4, e->vrec4, e->stream));
+            HIP_TRY(e, launch_f32_grid_sort(e->P, e->fa, e->key, e->rank, e->count, e->start, e->partials, e->rec4,
+                                            e->stream));
             ts.stop();
             Timed t(e, BS_K_PAIR);
-            HIP_TRY(e, launch_f32_grid_step(e->P, e->fa, e->fb, e->rec4, e->vrec4, e->key, e->start,
+            HIP_TRY(e, launch_f32_grid_step(e->P, e->fa, e->fb, e->rec4, e->key, e->rank, e->start, e->count,
                                             (float*)e->forces, e->digest, e->stream));
             t.stop();
             std::swap(e->fa, e->fb);

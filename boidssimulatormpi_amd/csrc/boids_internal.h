@@ -126,10 +126,6 @@ hipError_t launch_rows(Flocks F, const uint32_t* start, uint32_t* row_count, uin
 // sorted parts into its in-cell id order).
 hipError_t launch_scatter_ranked(uint32_t n, const uint32_t* key, const uint32_t* rank, const uint32_t* start,
                                  const uint32_t* id, uint32_t* perm, uint32_t* permid, hipStream_t stream);
-// The run sort alone: every run of 64 slots of perm / permid (boid index /
-// id, grouped by cell key[perm]) sorted by (cell, id) in place.  perm and
-// permid may be one array where a boid's index is its id.
-hipError_t launch_sort_runs(uint32_t n, const uint32_t* key, uint32_t* perm, uint32_t* permid, hipStream_t stream);
 // lat (mixed) receives the lattice copy; rec (FP64 grid) the records the
 // neighbour kernel fetches, three planes of n double2: (x, y), (z, vx), (vy, vz).
 hipError_t launch_gather(Flocks F, const uint32_t* perm, const uint32_t* permid, const uint32_t* key,
@@ -149,14 +145,16 @@ hipError_t launch_nbr_mixed(Flocks F, int nb, int tile, int max_cols, StateF64 i
                             uint32_t* count, double* forces, uint64_t* digest, uint32_t* recheck,
                             hipStream_t stream);
 hipError_t launch_copy(const void* src, void* dst, uint64_t bytes, hipStream_t stream);
-// Reference-faithful float grid (boids_f32grid.hip): the cell list of the
-// float state (keys, counting sort by (cell, id), sorted records), then the
-// step from it (id order in, id order out).
-hipError_t launch_f32_grid_sort(const DevParams& P, StateF32 st, uint32_t* key, uint32_t* rank, uint32_t* count,
-                                uint32_t* start, uint32_t* partials, uint32_t* perm, float4* rec, float4* vrec,
-                                hipStream_t stream);
-hipError_t launch_f32_grid_step(const DevParams& P, StateF32 in, StateF32 out, const float4* rec,
-                                const float4* vrec, const uint32_t* key, const uint32_t* start, float* forces,
+// Reference-faithful float grid (boids_f32grid.hip): cell keys, arrival ranks
+// and counts of a state from outside; the cell list from them (start, records);
+// the step from it (id order in, id order out), which leaves keys, ranks and
+// counts of the state it writes.
+hipError_t launch_f32_hash(const DevParams& P, StateF32 st, uint32_t* key, uint32_t* rank, uint32_t* count,
+                           hipStream_t stream);
+hipError_t launch_f32_grid_sort(const DevParams& P, StateF32 st, const uint32_t* key, const uint32_t* rank,
+                                uint32_t* count, uint32_t* start, uint32_t* partials, float4* rec, hipStream_t stream);
+hipError_t launch_f32_grid_step(const DevParams& P, StateF32 in, StateF32 out, const float4* rec, uint32_t* key,
+                                uint32_t* rank, const uint32_t* start, uint32_t* count, float* forces,
                                 uint64_t* digest, hipStream_t stream);
 // flock metrics (boids_metrics.hip)
 size_t metrics_workspace_bytes(uint32_t n, int G);

@@ -508,6 +508,16 @@ hipError_t launch_rows(Flocks F, const uint32_t* start, uint32_t* row_count, uin
     return hipGetLastError();
 }
 
+static hipError_t launch_sort_runs(uint32_t n, const uint32_t* key, uint32_t* perm, uint32_t* permid, hipStream_t stream)
+{
+    if (n == 0) return hipSuccess;
+    if (n <= (1u << 26))
+        hipLaunchKernelGGL(k_sort_runs<uint32_t>, dim3(blocks_for(n)), dim3(kBlock), 0, stream, n, key, perm, permid);
+    else
+        hipLaunchKernelGGL(k_sort_runs<uint64_t>, dim3(blocks_for(n)), dim3(kBlock), 0, stream, n, key, perm, permid);
+    return hipGetLastError();
+}
+
 hipError_t launch_scatter_ranked(uint32_t n, const uint32_t* key, const uint32_t* rank, const uint32_t* start,
                                  const uint32_t* id, uint32_t* perm, uint32_t* permid, hipStream_t stream)
 {
@@ -517,16 +527,6 @@ hipError_t launch_scatter_ranked(uint32_t n, const uint32_t* key, const uint32_t
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
     return launch_sort_runs(n, key, perm, permid, stream);
-}
-
-hipError_t launch_sort_runs(uint32_t n, const uint32_t* key, uint32_t* perm, uint32_t* permid, hipStream_t stream)
-{
-    if (n == 0) return hipSuccess;
-    if (n <= (1u << 26))
-        hipLaunchKernelGGL(k_sort_runs<uint32_t>, dim3(blocks_for(n)), dim3(kBlock), 0, stream, n, key, perm, permid);
-    else
-        hipLaunchKernelGGL(k_sort_runs<uint64_t>, dim3(blocks_for(n)), dim3(kBlock), 0, stream, n, key, perm, permid);
-    return hipGetLastError();
 }
 
 hipError_t launch_gather(Flocks F, const uint32_t* perm, const uint32_t* permid, const uint32_t* key,
