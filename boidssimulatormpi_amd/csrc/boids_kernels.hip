@@ -184,6 +184,81 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_tiles(uint32_t* count, ui
     if (threadIdx.x == 0) partials[blockIdx.x] = total;
 }
 
+// The whole scan in one workgroup, up to TILES tiles: every thread loads its
+// four counters of each tile at once, the waves scan theirs, and one wave
+// scans the waves' totals of all tiles -- two barriers whatever TILES is.
+template <int TILES>
+__global__ __launch_bounds__(kScanThreads) void k_scan_small(uint32_t* count, uint32_t* start, uint32_t m)
+{
+    static_assert(kScanItems == 4 && kScanThreads == 1024, "16-byte loads, 16 waves");
+    __shared__ uint32_t wsum[TILES * 16];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint4 v[TILES];
+    uint32_t in[TILES];
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+        const uint32_t at = (uint32_t)t * kScanTile + threadIdx.x * 4;
+        v[t] = make_uint4(0, 0, 0, 0);
+        if (at + 4 <= m) v[t] = *(const uint4*)(count + at);
+        else if (at < m) {
+            v[t].x = count[at];
+            if (at + 1 < m) v[t].y = count[at + 1];
+            if (at + 2 < m) v[t].z = count[at + 2];
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+        const uint32_t s = v[t].x + v[t].y + v[t].z + v[t].w;
+        uint32_t x = s;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t y = __shfl_up(x, d, 64);
+            if (lane >= (uint32_t)d) x += y;
+        }
+        if (lane == 63) wsum[16 * t + wave] = x;
+        in[t] = x - s;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        constexpr int PER = (TILES * 16 + 63) / 64;
+        uint32_t w[PER], sum = 0;
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const uint32_t at = lane * PER + k;
+            w[k] = at < TILES * 16 ? wsum[at] : 0u;
+            sum += w[k];
+        }
+        uint32_t x = sum;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t y = __shfl_up(x, d, 64);
+            if (lane >= (uint32_t)d) x += y;
+        }
+        x -= sum;
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const uint32_t at = lane * PER + k;
+            if (at < TILES * 16) wsum[at] = x;
+            x += w[k];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+        const uint32_t at = (uint32_t)t * kScanTile + threadIdx.x * 4;
+        const uint32_t r = in[t] + wsum[16 * t + wave];
+        const uint4 o = make_uint4(r, r + v[t].x, r + v[t].x + v[t].y, r + v[t].x + v[t].y + v[t].z);
+        if (at + 4 <= m) {
+            *(uint4*)(start + at) = o;
+            *(uint4*)(count + at) = make_uint4(0, 0, 0, 0);
+        } else if (at < m) {
+            start[at] = o.x; count[at] = 0u;
+            if (at + 1 < m) { start[at + 1] = o.y; count[at + 1] = 0u; }
+            if (at + 2 < m) { start[at + 2] = o.z; count[at + 2] = 0u; }
+        }
+    }
+}
+
 __global__ __launch_bounds__(kScanThreads) void k_scan_partials(uint32_t* partials, uint32_t nt)
 {
     __shared__ uint32_t wsum[17];
@@ -198,10 +273,22 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_partials(uint32_t* partia
     }
 }
 
+// Adds to every tile the totals of the tiles before it: partials[] holds the
+// totals themselves (SUM; each workgroup then adds up the ones before its own)
+// or their exclusive scan.
+template <bool SUM>
 __global__ __launch_bounds__(kScanThreads) void k_scan_add(uint32_t* start, uint32_t m,
                                                             const uint32_t* partials)
 {
-    const uint32_t add = partials[blockIdx.x];
+    __shared__ uint32_t wsum[17];
+    uint32_t add = 0;
+    if (SUM) {
+        uint32_t mine = 0;
+        for (uint32_t t = threadIdx.x; t < blockIdx.x; t += kScanThreads) mine += partials[t];
+        block_exclusive_scan(mine, wsum, &add);
+    } else {
+        add = partials[blockIdx.x];
+    }
     const uint32_t base = blockIdx.x * kScanTile + threadIdx.x * kScanItems;
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) {
@@ -475,15 +562,31 @@ hipError_t launch_hash_count(Flocks F, StateF64 st, uint32_t* key, uint32_t* ran
     return hipGetLastError();
 }
 
+// By size: one workgroup up to 8 tiles (13825 counters: 4.8 us, three launches
+// took 13; a workgroup's loads of 128 KB cost about a launch, so more tiles go
+// to more workgroups); beyond that two launches, the second adding up the totals of the tiles before each tile
+// itself, while these are few enough to read in a turn or two; else three.
+// count and start are 16-byte aligned.
 hipError_t launch_scan(uint32_t* count, uint32_t* start, uint32_t m, uint32_t* partials,
                        hipStream_t stream)
 {
     const uint32_t nt = (m + kScanTile - 1) / kScanTile;
-    hipLaunchKernelGGL(k_scan_tiles, dim3(nt), dim3(kScanThreads), 0, stream, count, start, m, partials);
-    if (nt <= 1) return hipGetLastError();      // one tile: its local scan is the scan
-    hipLaunchKernelGGL(k_scan_partials, dim3(1), dim3(kScanThreads), 0, stream, partials, nt);
-    hipLaunchKernelGGL(k_scan_add, dim3(nt), dim3(kScanThreads), 0, stream, start, m,
-                       (const uint32_t*)partials);
+    const dim3 one(1), tiles(nt), threads(kScanThreads);
+    if (nt <= 1) {
+        hipLaunchKernelGGL(k_scan_small<1>, one, threads, 0, stream, count, start, m);
+    } else if (nt <= 4) {
+        hipLaunchKernelGGL(k_scan_small<4>, one, threads, 0, stream, count, start, m);
+    } else if (nt <= 8) {
+        hipLaunchKernelGGL(k_scan_small<8>, one, threads, 0, stream, count, start, m);
+    } else {
+        hipLaunchKernelGGL(k_scan_tiles, tiles, threads, 0, stream, count, start, m, partials);
+        if (nt <= 2 * kScanThreads) {
+            hipLaunchKernelGGL(k_scan_add<true>, tiles, threads, 0, stream, start, m, (const uint32_t*)partials);
+        } else {
+            hipLaunchKernelGGL(k_scan_partials, one, threads, 0, stream, partials, nt);
+            hipLaunchKernelGGL(k_scan_add<false>, tiles, threads, 0, stream, start, m, (const uint32_t*)partials);
+        }
+    }
     return hipGetLastError();
 }
 
