@@ -39,14 +39,16 @@ __device__ __forceinline__ R norm3(R x, R y, R z)
     return sqrt(s);
 }
 
-// Per-axis minimum image of src/boid_simulation.cpp:164-178: the float
-// difference is compared in double against F/2; the shifted value is
-// rounded back to R.
+// Per-axis minimum image of src/boid_simulation.cpp:164-178: the difference
+// is compared with F/2 (in double there; half is F/2 for double and the
+// largest float not above it for float, which no float lies between), and
+// the shifted value is rounded back to R.
 template <typename R>
-__device__ __forceinline__ R min_image(R q, R p, double F, double half)
+__device__ __forceinline__ R min_image(R q, R p, double F, R half)
 {
-    if ((double)(q - p) > half) return (R)((double)q - F);
-    if ((double)(p - q) > half) return (R)((double)q + F);
+    const R d = q - p;
+    if (d > half) return (R)((double)q - F);
+    if (-d > half) return (R)((double)q + F);
     return q;
 }
 
@@ -56,6 +58,8 @@ template <> struct Th<float> {
     __device__ static float c(const DevParams& P, int r) { return P.c_thr_f[r]; }
     __device__ static float smax(const DevParams& P) { return P.s_max_f; }
     __device__ static float w(const DevParams& P, int r) { return P.w_f[r]; }
+    __device__ static float half(const DevParams& P) { return P.half_f; }
+    __device__ static float reach(const DevParams& P) { return P.s_reach_f; }
     __device__ static float vmax(const DevParams& P) { return P.vmax_f; }
     __device__ static float vmin(const DevParams& P) { return P.vmin_f; }
 };
@@ -64,6 +68,8 @@ template <> struct Th<double> {
     __device__ static double c(const DevParams& P, int r) { return P.c_thr[r]; }
     __device__ static double smax(const DevParams& P) { return P.s_max; }
     __device__ static double w(const DevParams& P, int r) { return P.w[r]; }
+    __device__ static double half(const DevParams& P) { return P.half; }
+    __device__ static double reach(const DevParams& P) { return P.s_reach; }
     __device__ static double vmax(const DevParams& P) { return P.vmax; }
     __device__ static double vmin(const DevParams& P) { return P.vmin; }
 };
@@ -243,5 +249,166 @@ __device__ __forceinline__ void exact_decide(const DevParams& P, double px, doub
     }
 }
 
+
+// ---------------------------------------------------------------------------
+// Reference-order steps (all-pairs, float grid): one wave per owner.
+// ---------------------------------------------------------------------------
+// Orders this wave's LDS writes before its later LDS reads (a wave's LDS
+// operations execute in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <typename R>
+__device__ __forceinline__ R lane_value(R v, uint32_t l)
+{
+    if constexpr (sizeof(R) == 4) {
+        return __builtin_bit_cast(R, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), (int)l));
+    } else {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v);
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, (int)l);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), (int)l);
+        return __builtin_bit_cast(R, ((uint64_t)hi << 32) | lo);
+    }
+}
+
+// 64-bit sum over the wave (butterfly), in every lane.
+__device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v)
+{
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)v, d, 64);
+        const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(v >> 32), d, 64);
+        v += ((uint64_t)hi << 32) | lo;
+    }
+    return v;
+}
+
+// Squared distance of the periodic images nearest each other, with one
+// rounding for the shift: below reach_of() for every pair within the largest
+// radius (a filter; the decisions take the reference's arithmetic).
+template <typename R>
+__device__ __forceinline__ R near2(R dx, R dy, R dz, R F, R inv_F)
+{
+    if constexpr (sizeof(R) == 4) {
+        dx = fmaf(-F, rintf(dx * inv_F), dx); dy = fmaf(-F, rintf(dy * inv_F), dy); dz = fmaf(-F, rintf(dz * inv_F), dz);
+        return fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+    } else {
+        dx = fma(-F, rint(dx * inv_F), dx); dy = fma(-F, rint(dy * inv_F), dy); dz = fma(-F, rint(dz * inv_F), dz);
+        return fma(dz, dz, fma(dy, dy, dx * dx));
+    }
+}
+
+// near2's bound for an owner.  Th<R>::reach allows for the rounding of
+// coordinates within 4 F (an owner within 2 F and a boid at most one image
+// away); an owner farther out takes every finite distance.
+template <typename R>
+__device__ __forceinline__ R reach_of(const DevParams& P, R px, R py, R pz)
+{
+    const R lim = 2 * (R)P.F;
+    return fabs(px) <= lim && fabs(py) <= lim && fabs(pz) <= lim ? Th<R>::reach(P) : (R)INFINITY;
+}
+
+// The sums of one owner in the reference's order.  add() takes up to 64 boids
+// in ascending id, one per lane: the lanes read their states, take the three
+// rule decisions of src/boid.cpp:27-42 with the exact thresholds (s < s_thr
+// <=> sqrt(s) < r; c >= c_thr && c <= 1 <=> acos(c) <= pi a) and write the
+// pairs' nine terms (src/boid_simulation.cpp:153-212) to an LDS table, 0 where
+// a rule does not hold; lane c < 9 then adds column c of the table.  A running
+// sum that starts at +0 is never -0, so adding +0 leaves it unchanged bit for
+// bit.  The columns are kStride words apart, so the nine lanes' 16-byte reads
+// take different banks.
+template <typename R>
+struct OrderedSums {
+    static constexpr uint32_t kStride = 64 + 16 / sizeof(R);
+    struct __align__(16) Terms { R v[9][kStride]; };
+    R sum = 0;                                          // lane c < 9: term c
+    int nc = 0, ns = 0, na = 0;
+    uint64_t hc = 0, hs = 0, ha = 0;                    // this lane's pairs' id hashes
+
+    template <typename St>
+    __device__ __forceinline__ void add(const DevParams& P, const St& in, R px, R py, R pz, R vx, R vy, R vz, R vn,
+                                        uint32_t lane, uint32_t boids, uint32_t j, Terms& terms, bool hash)
+    {
+        R t[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+        bool in_c = false, in_s = false, in_a = false;
+        if (lane < boids) {
+            const R h = Th<R>::half(P);
+            const R qx = min_image(in.x[j], px, P.F, h), qy = min_image(in.y[j], py, P.F, h),
+                    qz = min_image(in.z[j], pz, P.F, h);
+            const R ex = px - qx, ey = py - qy, ez = pz - qz;
+            const R s = ex * ex + ey * ey + ez * ez;
+            in_c = s < Th<R>::s(P, COH);
+            in_s = s < Th<R>::s(P, SEP);
+            in_a = s < Th<R>::s(P, ALI);
+            if ((in_c && P.cone[COH]) || (in_s && P.cone[SEP]) || (in_a && P.cone[ALI])) {
+                const R gx = qx - px, gy = qy - py, gz = qz - pz;
+                const R dot = vx * gx + vy * gy + vz * gz;
+                const R c = dot / (vn * sqrt(s));
+                if (P.cone[COH]) in_c = in_c && c >= Th<R>::c(P, COH) && c <= (R)1;
+                if (P.cone[SEP]) in_s = in_s && c >= Th<R>::c(P, SEP) && c <= (R)1;
+                if (P.cone[ALI]) in_a = in_a && c >= Th<R>::c(P, ALI) && c <= (R)1;
+            }
+            if (in_c) { t[0] = qx; t[1] = qy; t[2] = qz; }
+            if (in_s) {
+                const R d = sqrt(s);
+                t[3] = ex / d; t[4] = ey / d; t[5] = ez / d;
+            }
+            if (in_a) { t[6] = in.vx[j]; t[7] = in.vy[j]; t[8] = in.vz[j]; }
+            if (hash) {
+                const uint64_t hh = mix64(j);
+                hc += in_c ? hh : 0; hs += in_s ? hh : 0; ha += in_a ? hh : 0;
+            }
+        }
+        nc += __popcll(__builtin_amdgcn_ballot_w64(in_c));
+        ns += __popcll(__builtin_amdgcn_ballot_w64(in_s));
+        na += __popcll(__builtin_amdgcn_ballot_w64(in_a));
+#pragma unroll
+        for (int k = 0; k < 9; ++k) terms.v[k][lane] = t[k];
+        wave_lds_order();
+        if (lane < 9) {
+            struct __align__(16) Four { R x, y, z, w; };
+            const Four* col = (const Four*)terms.v[lane];
+            const uint32_t cnt = (boids + 15) / 16;                 // the terms beyond them are 0
+            for (uint32_t l = 0; l < cnt; ++l) {
+                const Four a = col[4 * l], b = col[4 * l + 1], d = col[4 * l + 2], e = col[4 * l + 3];
+                sum += a.x; sum += a.y; sum += a.z; sum += a.w;
+                sum += b.x; sum += b.y; sum += b.z; sum += b.w;
+                sum += d.x; sum += d.y; sum += d.z; sum += d.w;
+                sum += e.x; sum += e.y; sum += e.z; sum += e.w;
+            }
+        }
+        wave_lds_order();
+    }
+    __device__ __forceinline__ R total(uint32_t c) const { return lane_value(sum, c); }
+    __device__ __forceinline__ void hash_sums() { hc = wave_sum_u64(hc); hs = wave_sum_u64(hs); ha = wave_sum_u64(ha); }
+};
+
+// Phase B (src/boid_simulation.cpp:216-248) of an owner from its nine sums
+// (cohesion, separation, alignment), and its forces and digest.
+template <typename R>
+__device__ __forceinline__ void finish_ordered(const DevParams& P, const OrderedSums<R>& S, const R (&t)[9], uint32_t i,
+                                               R& px, R& py, R& pz, R& vx, R& vy, R& vz, R* forces, uint64_t* digest)
+{
+    R scx = t[0], scy = t[1], scz = t[2], sax = t[6], say = t[7], saz = t[8];
+    if (S.nc != 0) { const R k = (R)S.nc; scx = scx / k - px; scy = scy / k - py; scz = scz / k - pz; }
+    if (S.na != 0) { const R k = (R)S.na; sax = sax / k - vx; say = say / k - vy; saz = saz / k - vz; }
+    const R wc = Th<R>::w(P, COH), ws = Th<R>::w(P, SEP), wa = Th<R>::w(P, ALI);
+    const R dx = (scx * wc + t[3] * ws) + sax * wa;
+    const R dy = (scy * wc + t[4] * ws) + say * wa;
+    const R dz = (scz * wc + t[5] * ws) + saz * wa;
+    if (forces) {
+        R* f = forces + 9 * (size_t)i;
+        f[0] = scx; f[1] = scy; f[2] = scz; f[3] = t[3]; f[4] = t[4]; f[5] = t[5]; f[6] = sax; f[7] = say; f[8] = saz;
+    }
+    if (digest) {
+        uint64_t* d = digest + 4 * (size_t)i;
+        d[0] = (uint64_t)S.nc | ((uint64_t)S.ns << 21) | ((uint64_t)S.na << 42);
+        d[1] = S.hc; d[2] = S.hs; d[3] = S.ha;
+    }
+    integrate<R>(P, px, py, pz, vx, vy, vz, dx, dy, dz);
+}
 
 }  // namespace boids

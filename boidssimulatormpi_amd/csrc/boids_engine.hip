@@ -203,6 +203,7 @@ struct bs_engine {
     Lattice lat{};
     double2* rec = nullptr;            // FP64 grid: interleaved pair records
     float4* rec4 = nullptr;            // float grid: positions and ids by cell
+    uint32_t* outside = nullptr;       // float grid: 1 once a boid of the state was outside the field
     uint32_t* recheck = nullptr;
     uint32_t* overflow = nullptr;      // chunk-table count beyond its capacity (0: none), in pinned host memory
     void* scratch = nullptr;           // this device's static scratch (allocation-free entry points)
@@ -392,6 +393,7 @@ static int derive_thresholds(const bs_params* p, DevParams* P, std::string* why)
     const double w[3] = {p->sep_w, p->ali_w, p->coh_w};
     P->F = p->field;
     P->half = p->field / 2;
+    P->half_f = round_down_f(P->half);
     P->s_max = -1.0;
     P->s_max_f = -1.0f;
     P->unit = p->field / 4294967296.0;
@@ -435,6 +437,12 @@ static int derive_thresholds(const bs_params* p, DevParams* P, std::string* why)
         P->c_hi[k] = P->cone[k] ? round_up_f(cth + beta_c) : -INFINITY;
         P->c_top[k] = P->cone[k] ? round_down_f(1.0 - beta_c) : INFINITY;
     }
+    // |q - p| carries 3 roundings of at most 2 F eps an axis, the reference's own
+    // arithmetic less than that again
+    const double reach_f = (sqrt((double)P->s_max_f) + 2e-6 * p->field) * (1.0 + 1e-5);
+    P->s_reach_f = round_up_f(reach_f * reach_f);
+    const double reach = (sqrt(P->s_max) + 1e-14 * p->field) * (1.0 + 1e-13);
+    P->s_reach = reach * reach * (1.0 + 1e-15);
     P->band_k = 8.0f;   // >= 2*sqrt(3) lattice units of displacement error, x2 margin
     P->same_cone = 1;
     for (int k = 1; k < 3; ++k)
@@ -795,9 +803,13 @@ static int create_engine(const bs_params* fp, uint32_t count, bool batch, bs_eng
             e->G = G;
             e->edge = p->field / G;
             e->P.G = G;
-            e->P.sx = 1;
+            // Half cells: the sphere around an owner then touches cells that hold a
+            // third of the boids of the 27 whole ones.  Where eight times the cells
+            // would outgrow the boids (8 counters each) or 32 bits, whole ones.
+            const uint64_t half = 8ull * G * G * G;
+            e->P.sx = half < (1ull << 31) && half <= std::max<uint64_t>(8ull * e->prm.n, 1u << 15) ? 2 : 1;
             e->P.inv_edge = G / p->field;
-            e->ncell1 = (uint32_t)((uint64_t)G * G * G + 1);
+            e->ncell1 = (uint32_t)((uint64_t)G * G * G * (e->P.sx == 2 ? 8 : 1) + 1);
         }
     }
 
@@ -825,7 +837,8 @@ static int create_engine(const bs_params* fp, uint32_t count, bool batch, bs_eng
         const uint32_t ntiles = (e->ncell1 + 4095) / 4096;
         if ((rc = dev_alloc(e, &e->key, n)) || (rc = dev_alloc(e, &e->rank, n)) ||
             (rc = dev_alloc(e, &e->count, e->ncell1)) || (rc = dev_alloc(e, &e->start, e->ncell1)) ||
-            (rc = dev_alloc(e, &e->partials, ntiles)) || (rc = dev_alloc(e, &e->rec4, n)))
+            (rc = dev_alloc(e, &e->partials, ntiles)) || (rc = dev_alloc(e, &e->rec4, n)) ||
+            (rc = dev_alloc(e, &e->outside, 1)))
             return bail(rc);
         st = hipMemsetAsync(e->count, 0, sizeof(uint32_t) * e->ncell1, e->stream);
         if (st != hipSuccess) { hip_fail(e, st, "hipMemsetAsync"); return bail(BS_E_HIP); }
@@ -1178,7 +1191,8 @@ extern "C" int bs_set_state_f32(bs_engine* e, const float* xyzv6)
         HIP_TRY(e, launch_unpack(n, (const float*)e->tmp_pos, e->fa, e->stream));
         if (e->mode == BS_MODE_GRID_F32REF) {                // the last state's counts give way to this one's
             HIP_TRY(e, hipMemsetAsync(e->count, 0, sizeof(uint32_t) * e->ncell1, e->stream));
-            HIP_TRY(e, launch_f32_hash(e->P, e->fa, e->key, e->rank, e->count, e->stream));
+            HIP_TRY(e, hipMemsetAsync(e->outside, 0, sizeof(uint32_t), e->stream));
+            HIP_TRY(e, launch_f32_hash(e->P, e->fa, e->key, e->rank, e->count, e->outside, e->stream));
         }
         HIP_TRY(e, hipStreamSynchronize(e->stream));
         loan.reader = nullptr;
@@ -1398,7 +1412,7 @@ extern "C" int bs_step(bs_engine* e, uint32_t nsteps)
             ts.stop();
             Timed t(e, BS_K_PAIR);
             HIP_TRY(e, launch_f32_grid_step(e->P, e->fa, e->fb, e->rec4, e->key, e->rank, e->start, e->count,
-                                            (float*)e->forces, e->digest, e->stream));
+                                            e->outside, (float*)e->forces, e->digest, e->stream));
             t.stop();
             std::swap(e->fa, e->fb);
             break;

@@ -37,8 +37,9 @@ constexpr int kChunkSpanMax = 16;
 struct DevParams {
     uint32_t n;
     int32_t G;                 // cells per axis (grid modes); x has sx * G columns
-    int32_t sx;                // x columns per cell edge (grid modes): 1 or 2
+    int32_t sx;                // x columns (float grid: cells on every axis) per cell edge (grid modes): 1 or 2
     double F, half;            // field edge, F/2
+    float half_f;              // the largest float <= half
     double inv_edge;           // G / F (x columns: sx * G / F)
     // double-precision exact thresholds (FP64 modes and mixed rechecks)
     double s_thr[3];           // d < r  <=>  s < s_thr   (s = squared distance, no FMA)
@@ -48,6 +49,10 @@ struct DevParams {
     double vmax, vmin;
     // float exact thresholds (reference-faithful float mode)
     float s_thr_f[3], c_thr_f[3], s_max_f;
+    // bounds that no pair within the largest radius reaches by the filters'
+    // one-rounding distance (boids_device.h: near2)
+    float s_reach_f;
+    double s_reach;
     float w_f[3];
     float vmax_f, vmin_f;
     int32_t cone[3];           // 1: the rule has a view cone (a < 1); 0: distance only
@@ -148,14 +153,15 @@ hipError_t launch_copy(const void* src, void* dst, uint64_t bytes, hipStream_t s
 // Reference-faithful float grid (boids_f32grid.hip): cell keys, arrival ranks
 // and counts of a state from outside; the cell list from them (start, records);
 // the step from it (id order in, id order out), which leaves keys, ranks and
-// counts of the state it writes.
+// counts of the state it writes.  *outside becomes 1 once a boid of either
+// state lies outside the field (set to 0 with a state from outside).
 hipError_t launch_f32_hash(const DevParams& P, StateF32 st, uint32_t* key, uint32_t* rank, uint32_t* count,
-                           hipStream_t stream);
+                           uint32_t* outside, hipStream_t stream);
 hipError_t launch_f32_grid_sort(const DevParams& P, StateF32 st, const uint32_t* key, const uint32_t* rank,
                                 uint32_t* count, uint32_t* start, uint32_t* partials, float4* rec, hipStream_t stream);
 hipError_t launch_f32_grid_step(const DevParams& P, StateF32 in, StateF32 out, const float4* rec, uint32_t* key,
-                                uint32_t* rank, const uint32_t* start, uint32_t* count, float* forces,
-                                uint64_t* digest, hipStream_t stream);
+                                uint32_t* rank, const uint32_t* start, uint32_t* count, uint32_t* outside,
+                                float* forces, uint64_t* digest, hipStream_t stream);
 // flock metrics (boids_metrics.hip)
 size_t metrics_workspace_bytes(uint32_t n, int G);
 // What the static scratch is priced at: 64 bytes per boid and 8 per cell of a

@@ -29,19 +29,6 @@ namespace boids {
 // ---------------------------------------------------------------------------
 constexpr int kWaveOwners = kBlock / 64;     // owners (waves) per workgroup
 
-template <typename R>
-__device__ __forceinline__ R lane_value(R v, uint32_t l)
-{
-    if constexpr (sizeof(R) == 4) {
-        return __builtin_bit_cast(R, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), (int)l));
-    } else {
-        const uint64_t u = __builtin_bit_cast(uint64_t, v);
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, (int)l);
-        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), (int)l);
-        return __builtin_bit_cast(R, ((uint64_t)hi << 32) | lo);
-    }
-}
-
 template <typename R, typename St>
 __global__ __launch_bounds__(kBlock) void k_allpairs_wave(DevParams P, St in, St out, R* forces,
                                                           uint64_t* digest)
@@ -76,9 +63,9 @@ __global__ __launch_bounds__(kBlock) void k_allpairs_wave(DevParams P, St in, St
         bool in_c = false, in_s = false, in_a = false;
         R qx = 0, qy = 0, qz = 0, tx = 0, ty = 0, tz = 0, wx = 0, wy = 0, wz = 0;
         if (j < n && j != i) {
-            qx = min_image(cx, px, P.F, P.half);
-            qy = min_image(cy, py, P.F, P.half);
-            qz = min_image(cz, pz, P.F, P.half);
+            qx = min_image(cx, px, P.F, Th<R>::half(P));
+            qy = min_image(cy, py, P.F, Th<R>::half(P));
+            qz = min_image(cz, pz, P.F, Th<R>::half(P));
             const R ex = px - qx, ey = py - qy, ez = pz - qz;
             const R s = ex * ex + ey * ey + ez * ez;
             if (s < smax) {

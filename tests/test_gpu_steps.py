@@ -1,4 +1,5 @@
-"""The scan of the cell counts at the sizes where its way changes."""
+"""The reference-order step of the float grid and the scan of the cell
+counts at the sizes and positions where their ways change."""
 import numpy as np
 import pytest
 
@@ -22,6 +23,39 @@ def flock(n, far, seed):
         st[: n // 2, :3] = at[np.arange(n // 2) // 4] + 0.02 * g.random((n // 2, 3))
         st[n // 4, 0] = np.nan
     return st
+
+
+@pytest.mark.parametrize("n,cells", [(2, 3), (700, 3), (700, 4), (700, 16), (700, 17), (5000, 17), (4913, 17), (4912, 17)])
+@pytest.mark.parametrize("out", [False, True])
+def test_float_grid_half_and_whole_cells(n, cells, out):
+    # half cells up to 16 cells per axis or n = 17^3, whole ones beyond; clumps
+    # at the faces; boids a little outside the field (still within a cell edge of
+    # all their neighbours)
+    print(n, cells, out, flush=True)
+    g = np.random.default_rng(n + cells)
+    st = flock(n, False, n).astype(np.float32)
+    edge = g.choice([0.0, 0.01, 0.98, 0.999], (n // 2, 3)) + 0.001 * g.random((n // 2, 3))
+    st[: n // 2, :3] = edge
+    st[0, 0] = 1.0
+    if out:
+        st[: n // 8, g.integers(3)] = np.float32(-0.004)
+        st[n // 8: n // 4, g.integers(3)] = np.float32(1.004)
+    flags = E.FLAG_DIGEST | E.FLAG_FORCES
+    a = B.Engine(B.make_params(n, 1.0, **RULES, mode=E.MODE_ALLPAIRS_F32REF, flags=flags))
+    b = B.Engine(B.make_params(n, 1.0, **RULES, mode=E.MODE_GRID_F32REF, flags=flags, cells_per_axis=cells))
+    assert b.info().mode == E.MODE_GRID_F32REF and b.info().cells_per_axis == cells
+    for again in range(2):                             # the second state starts anew
+        for e in (a, b):
+            e.set_state(xyzv6=st)
+        for t in range(3):
+            for e in (a, b):
+                e.step(1)
+            assert np.array_equal(a.digest(), b.digest()), t
+            assert np.array_equal(a.forces_f32(), b.forces_f32()), t
+            assert all(np.array_equal(x, y) for x, y in zip(a.state_f32(), b.state_f32())), t
+        st = flock(n, False, n + 1).astype(np.float32)
+    a.close()
+    b.close()
 
 
 @pytest.mark.parametrize("cells", [3, 12, 15, 16, 20, 25, 26, 31, 32, 33, 60, 150, 210])
