@@ -1,10 +1,11 @@
-"""The reference-order step of the float grid and the scan of the cell
+"""The reference-order steps (all-pairs, float grid) and the scan of the cell
 counts at the sizes and positions where their ways change."""
 import numpy as np
 import pytest
 
 import boidssimulatormpi_amd as B
 from boidssimulatormpi_amd import engine as E
+from oracle import oracle as O
 
 from test_gpu_grid_build import check, single
 
@@ -23,6 +24,32 @@ def flock(n, far, seed):
         st[: n // 2, :3] = at[np.arange(n // 2) // 4] + 0.02 * g.random((n // 2, 3))
         st[n // 4, 0] = np.nan
     return st
+
+
+@pytest.mark.parametrize("mode", [E.MODE_ALLPAIRS_F32REF, E.MODE_ALLPAIRS_F64])
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 127, 128, 129, 1000])
+@pytest.mark.parametrize("far", [False, True])
+def test_allpairs_equals_oracle(mode, n, far):
+    # one batch, several, and their remainders; lists that fill in the middle of the flock
+    print(mode, n, far, flush=True)
+    f32 = mode == E.MODE_ALLPAIRS_F32REF
+    st = flock(n, far, n)
+    e = B.Engine(B.make_params(n, 1.0, **RULES, mode=mode, flags=E.FLAG_DIGEST))
+    if f32:
+        st = st.astype(np.float32)
+        e.set_state(xyzv6=st)
+    else:
+        e.set_state(pos=st[:, :3].copy(), vel=st[:, 3:].copy())
+    p, v = st[:, :3].copy(), st[:, 3:].copy()
+    with np.errstate(invalid="ignore"):
+        for t in range(2):
+            _, d = O.step(O.params(1.0, **RULES), p, v, digest=True)
+            e.step(1)
+            gp, gv = e.state_f32() if f32 else e.state_f64()
+            # the same operations in the same order
+            assert np.array_equal(e.digest(), d), t
+            assert np.array_equal(gp, p, equal_nan=True) and np.array_equal(gv, v, equal_nan=True), t
+    e.close()
 
 
 @pytest.mark.parametrize("n,cells", [(2, 3), (700, 3), (700, 4), (700, 16), (700, 17), (5000, 17), (4913, 17), (4912, 17)])
