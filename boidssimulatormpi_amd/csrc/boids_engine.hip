@@ -24,7 +24,7 @@
 #endif
 static_assert(BS_MIXED_SUBX >= 1 && BS_MIXED_SUBX <= boids::kSubXMax && BS_F64_SUBX >= 1 &&
                   BS_F64_SUBX <= boids::kSubXMax, "x columns per cell edge");
-// Most x columns a neighbour-kernel chunk covers (k_rows_pass cuts runs of
+// Most x columns a neighbour-kernel chunk covers (rows_pass cuts runs of
 // boids short there): narrow chunks give the lanes of a wave windows of more
 // equal length (phase 1 runs as long as the longest), wide ones fewer tile
 // restagings; measured best for both paths: 12 half-columns (6 cell edges).
@@ -759,7 +759,7 @@ static int create_engine(const bs_params* fp, uint32_t count, bool batch, bs_eng
             const uint32_t ng = (Gx + kSpanMax - 1) / kSpanMax;
             d.span = (Gx + ng - 1) / ng;
             // chunk-table slack per span group: its last chunk, plus one chunk
-            // cut short per cspan columns (k_rows_pass)
+            // cut short per cspan columns (rows_pass)
             e->groups += (uint64_t)G * G * ((Gx + d.span - 1) / d.span) * (1 + (d.span - 1) / e->cspan);
             e->max_span = std::max(e->max_span, (int)d.span);
             cells += (uint64_t)Gx * G * G;
@@ -844,7 +844,7 @@ static int create_engine(const bs_params* fp, uint32_t count, bool batch, bs_eng
         if (st != hipSuccess) { hip_fail(e, st, "hipMemsetAsync"); return bail(BS_E_HIP); }
     }
     if (is_grid(e->mode)) {
-        // full chunks <= n / chunk; groups counts each (row, span group)'s last chunk and short cuts (k_rows_pass)
+        // full chunks <= n / chunk; groups counts each (row, span group)'s last chunk and short cuts (rows_pass)
         if ((uint64_t)(n + e->chunk - 1) / e->chunk + e->groups + 1 > 0x7fffffffull) return bail(fail(e, BS_E_ARG, "chunk table too large"));
         e->max_chunks = (uint32_t)((n + e->chunk - 1) / e->chunk + e->groups + 1);
         const uint32_t ntiles = (e->ncell1 + 4095) / 4096;
@@ -967,12 +967,11 @@ static int grid_sort_into_a(bs_engine* e)
 {
     Timed t(e, BS_K_SCAN);
     HIP_TRY(e, launch_scan(e->count, e->start, e->ncell1, e->partials, e->stream));
-    HIP_TRY(e, launch_rows(flock_view(e), e->start, e->row_count, e->row_off, e->partials, e->table, e->nchunks,
-                           e->max_chunks, e->overflow,
-                           (int)e->chunk, e->cspan, e->sx * e->max_g, e->stream));
     t.stop();
     Timed t2(e, BS_K_SCATTER);
-    HIP_TRY(e, launch_scatter_ranked(e->prm.n, e->key, e->rank, e->start, e->db.id, e->perm, e->permid, e->stream));
+    const Rows rows{e->row_count, e->table, e->nchunks, e->overflow, e->chunk, (uint32_t)e->cspan, e->max_chunks};
+    HIP_TRY(e, launch_scatter_ranked(flock_view(e), rows, e->sx * e->max_g, e->row_off, e->partials, e->key, e->rank,
+                                     e->start, e->db.id, e->perm, e->permid, e->stream));
     t2.stop();
     Timed t3(e, BS_K_GATHER);
     HIP_TRY(e, launch_gather(flock_view(e), e->perm, e->permid, e->key, e->start, e->count, e->db, e->da,
@@ -1205,7 +1204,7 @@ extern "C" int bs_set_state_f32(bs_engine* e, const float* xyzv6)
     return settle_state(e, st, loan);
 }
 
-// Reports a chunk table cut short by its capacity (k_rows_pass clamps the
+// Reports a chunk table cut short by its capacity (rows_pass clamps the
 // count and leaves the full one in e->overflow): the update then skipped
 // boids, so the state is not a valid result.  The capacity bound makes this
 // unreachable; the check runs wherever the host reads results back.

@@ -120,17 +120,26 @@ hipError_t launch_hash_count(Flocks F, StateF64 st, uint32_t* key, uint32_t* ran
                              hipStream_t stream);
 hipError_t launch_scan(uint32_t* count, uint32_t* start, uint32_t n, uint32_t* partials,
                        hipStream_t stream);
-// chunk = most boids per chunk, cspan = most x columns a chunk covers,
-// max_cols = x columns of the longest row (sx * G over the flocks), cap =
-// entries `table` holds (a count beyond it is clamped and left in *overflow).
-hipError_t launch_rows(Flocks F, const uint32_t* start, uint32_t* row_count, uint32_t* row_off,
-                       uint32_t* partials, uint4* table, uint32_t* nchunks, uint32_t cap, uint32_t* overflow,
-                       int chunk, int cspan, int max_cols, hipStream_t stream);
-// Scatter by the arrival ranks the counting pass recorded (no atomics),
-// then sort every run of 64 slots by (cell, id) (the gather merges a cell's
-// sorted parts into its in-cell id order).
-hipError_t launch_scatter_ranked(uint32_t n, const uint32_t* key, const uint32_t* rank, const uint32_t* start,
-                                 const uint32_t* id, uint32_t* perm, uint32_t* permid, hipStream_t stream);
+// The chunk table of the neighbour kernels: chunk = most boids per chunk,
+// cspan = most x columns a chunk covers, cap = entries `table` holds (a count
+// beyond it is clamped and left in *overflow), count = chunks per row
+// (16-byte aligned); the rest is the launcher's.
+struct Rows {
+    uint32_t* count;
+    uint4* table;
+    uint32_t *nchunks, *overflow;
+    uint32_t chunk, cspan, cap;
+    const uint32_t* off;       // offsets of the rows' chunks, or null
+    uint32_t stride, blocks;   // LDS words per row, workgroups of the rows
+};
+// Scatter by the arrival ranks the counting pass recorded (no atomics), then
+// sort every run of 64 slots by (cell, id) (the gather merges a cell's sorted
+// parts into its in-cell id order), and the chunk table.  max_cols = x columns
+// of the longest row (sx * G over the flocks); row_off and partials: scratch
+// of the rows' scan.
+hipError_t launch_scatter_ranked(Flocks F, Rows R, int max_cols, uint32_t* row_off, uint32_t* partials,
+                                 const uint32_t* key, const uint32_t* rank, const uint32_t* start, const uint32_t* id,
+                                 uint32_t* perm, uint32_t* permid, hipStream_t stream);
 // lat (mixed) receives the lattice copy; rec (FP64 grid) the records the
 // neighbour kernel fetches, three planes of n double2: (x, y), (z, vx), (vy, vz).
 hipError_t launch_gather(Flocks F, const uint32_t* perm, const uint32_t* permid, const uint32_t* key,

@@ -256,34 +256,47 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_add(uint32_t* start, uint
 // most (span - 1) / cspan of them: the table holds at most n / chunk +
 // groups * (1 + (span - 1) / cspan) entries.  One wave per row: the
 // row's column starts are read into LDS (coalesced) and one lane walks them.
-// Pass 1 counts the row's chunks; after a scan of the counts, pass 2 writes
-// them at the row's offset (rows in order: neighbouring rows' chunks stay
-// adjacent in the table).
-constexpr int kRowWaves = 4;
-
+// Pass 1 counts the row's chunks; pass 2 writes them after those of the rows
+// before it (rows in order: neighbouring rows' chunks stay adjacent in the
+// table).
+// The passes are the first workgroups of the two kernels that sort the boids
+// (k_scatter_ranked, k_sort_runs), which need nothing of them: a launch of its
+// own costs about 4.5 us whatever it does.  While the rows are few (kRowsSum),
+// pass 2 adds up the counts of the rows before its own; beyond that a scan
+// between the two kernels leaves the offsets in `off`.
+// One update, own launches / shared: FP64 N = 16384 159 / 152 us, mixed N = 50021
+// 83 / 76, mixed N = 2^20 506 / 491, mixed N = 2^22 4525 / 4490 (6241 rows), 64
+// flocks of 16384 735 / 726 (9216 rows).  At kRowsSum the sums read 134 MB of
+// cached counts, about what the scan's launches cost.
 //
 // The bound is the table's capacity (`cap`); pass 2 writes no entry at or
 // beyond it, and should the count ever exceed it, *nchunks is clamped to
 // the capacity and the full count is left in *overflow (non-zero marks the
 // table as cut short; the host reports it as an error).
+constexpr int kRowWaves = kBlock / 64;
+constexpr uint32_t kRowsSum = 16384;
+
 template <bool WRITE>
-__global__ __launch_bounds__(64 * kRowWaves) void k_rows_pass(Flocks F, const uint32_t* __restrict__ start,
-                                                              uint32_t* row_count, const uint32_t* row_off,
-                                                              uint4* table, uint32_t* nchunks, uint32_t chunk,
-                                                              uint32_t cspan, uint32_t stride, uint32_t cap,
-                                                              uint32_t* overflow)
+__device__ __forceinline__ void rows_pass(const Flocks& F, const Rows& R, const uint32_t* __restrict__ start)
 {
     extern __shared__ uint32_t rs[];            // kRowWaves x stride (>= the longest row's columns + 1)
+    __shared__ uint32_t wsum[kRowWaves];
     const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-    const uint32_t r = blockIdx.x * kRowWaves + w;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        if (WRITE) {
-            const uint32_t total = row_off[F.rows];
-            *nchunks = min(total, cap);
-            if (total > cap) *overflow = total;
-        } else {
-            row_count[F.rows] = 0u;             // the scan's total lands in row_off[rows]
+    const uint32_t r0 = blockIdx.x * kRowWaves, r = r0 + w;
+    uint32_t before = 0;                        // chunks of the rows before r
+    if (WRITE && !R.off) {
+        for (uint32_t q = threadIdx.x; q < r0 / 4; q += kBlock) {     // (kRowWaves = 4: whole quads)
+            const uint4 c = ((const uint4*)R.count)[q];
+            before += c.x + c.y + c.z + c.w;
         }
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) before += __shfl_xor(before, d, 64);
+        if (lane == 0) wsum[w] = before;
+        __syncthreads();
+        before = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+        for (uint32_t q = r0; q < min(r, F.rows); ++q) before += R.count[q];
+    } else if (WRITE && r < F.rows) {
+        before = R.off[r];
     }
     if (r >= F.rows) return;                    // whole waves only: no barrier follows
     const uint32_t f = F.row_flock ? F.row_flock[r] : 0u;
@@ -291,37 +304,44 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_rows_pass(Flocks F, const ui
     const uint32_t G = (uint32_t)fd.P.sx * (uint32_t)fd.P.G, span = fd.span;   // x columns of the row
     const uint32_t rl = r - fd.row_base;
     const uint32_t c0 = fd.cell_base + rl * G;
-    uint32_t* cs = rs + w * stride;
+    uint32_t* cs = rs + w * R.stride;
     for (uint32_t x = lane; x <= G; x += 64) cs[x] = start[c0 + x];
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     if (lane != 0) return;
-    uint32_t k = WRITE ? row_off[r] : 0u;
+    uint32_t k = before;
     for (uint32_t x0 = 0; x0 < G; x0 += span) {
         const uint32_t x1 = min(G, x0 + span);
         const uint32_t hi = cs[x1];
         uint32_t t0 = cs[x0], xa = x0;
         while (t0 < hi) {
             while (cs[xa + 1] <= t0) ++xa;          // cell of boid t0
-            uint32_t t1 = min(hi, t0 + chunk);
-            if (xa + cspan < x1) t1 = min(t1, cs[xa + cspan]);
-            if (WRITE && k < cap) table[k] = make_uint4(rl, t0, t1, f);
+            uint32_t t1 = min(hi, t0 + R.chunk);
+            if (xa + R.cspan < x1) t1 = min(t1, cs[xa + R.cspan]);
+            if (WRITE && k < R.cap) R.table[k] = make_uint4(rl, t0, t1, f);
             ++k;
             t0 = t1;
         }
     }
-    if (!WRITE) row_count[r] = k;
+    if (!WRITE) {
+        R.count[r] = k;
+    } else if (r + 1 == F.rows) {
+        *R.nchunks = min(k, R.cap);
+        if (k > R.cap) *R.overflow = k;
+    }
 }
 
-__global__ __launch_bounds__(kBlock) void k_scatter_ranked(uint32_t n, const uint32_t* __restrict__ key,
+// The first R.blocks workgroups count the rows' chunks.
+__global__ __launch_bounds__(kBlock) void k_scatter_ranked(Flocks F, Rows R, const uint32_t* __restrict__ key,
                                                            const uint32_t* __restrict__ rank,
                                                            const uint32_t* __restrict__ start,
                                                            const uint32_t* __restrict__ id, uint32_t* perm,
                                                            uint32_t* permid)
 {
-    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
-    if (s >= n) return;
+    if (blockIdx.x < R.blocks) { rows_pass<false>(F, R, start); return; }
+    const uint32_t s = (blockIdx.x - R.blocks) * kBlock + threadIdx.x;
+    if (s >= F.n) return;
     const uint32_t t = start[key[s]] + rank[s];
     perm[t] = s;
     permid[t] = id[s];
@@ -334,7 +354,8 @@ __global__ __launch_bounds__(kBlock) void k_scatter_ranked(uint32_t n, const uin
 // spanning runs leaves one ascending part per run, which k_gather merges.
 // Keys are 32-bit (6-bit part index, 26-bit id) when every id is below 2^26,
 // else 64-bit.  A run already in order (the common case: boids arriving from
-// one old cell are ranked in lane order) is left alone.
+// one old cell are ranked in lane order) is left alone.  The first R.blocks
+// workgroups write the rows' chunks.
 template <typename K>
 __device__ __forceinline__ K shfl_xor_key(K v, uint32_t m)
 {
@@ -347,12 +368,14 @@ __device__ __forceinline__ K shfl_xor_key(K v, uint32_t m)
 }
 
 template <typename K>
-__global__ __launch_bounds__(kBlock) void k_sort_runs(uint32_t n, const uint32_t* __restrict__ key,
-                                                      uint32_t* perm, uint32_t* permid)
+__global__ __launch_bounds__(kBlock) void k_sort_runs(Flocks F, Rows R, const uint32_t* __restrict__ key,
+                                                      const uint32_t* __restrict__ start, uint32_t* perm,
+                                                      uint32_t* permid)
 {
-    const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
+    if (blockIdx.x < R.blocks) { rows_pass<true>(F, R, start); return; }
+    const uint32_t t = (blockIdx.x - R.blocks) * kBlock + threadIdx.x;
     const uint32_t lane = threadIdx.x & 63u;
-    const bool in = t < n;
+    const bool in = t < F.n;
     uint32_t p = 0u, id = 0u, c = 0xFFFFFFFFu;
     if (in) {
         p = perm[t];
@@ -539,46 +562,30 @@ hipError_t launch_scan(uint32_t* count, uint32_t* start, uint32_t m, uint32_t* p
     return hipGetLastError();
 }
 
-hipError_t launch_rows(Flocks F, const uint32_t* start, uint32_t* row_count, uint32_t* row_off,
-                       uint32_t* partials, uint4* table, uint32_t* nchunks, uint32_t cap, uint32_t* overflow,
-                       int chunk, int cspan, int max_cols, hipStream_t stream)
+hipError_t launch_scatter_ranked(Flocks F, Rows R, int max_cols, uint32_t* row_off, uint32_t* partials,
+                                 const uint32_t* key, const uint32_t* rank, const uint32_t* start, const uint32_t* id,
+                                 uint32_t* perm, uint32_t* permid, hipStream_t stream)
 {
-    if (F.count == 0 || chunk <= 0 || F.rows == 0 || cspan < 1 || cspan > kChunkSpanMax || max_cols < 1 ||
+    if (F.count == 0 || R.chunk == 0 || F.rows == 0 || R.cspan < 1 || R.cspan > kChunkSpanMax || max_cols < 1 ||
         max_cols > kSubXMax * kMaxCells)
         return hipErrorInvalidValue;
-    const dim3 grid((F.rows + kRowWaves - 1) / kRowWaves);
-    const uint32_t stride = (uint32_t)max_cols + 1;
-    const size_t dyn = sizeof(uint32_t) * kRowWaves * stride;
-    hipLaunchKernelGGL(k_rows_pass<false>, grid, dim3(64 * kRowWaves), dyn, stream, F, start, row_count,
-                       (const uint32_t*)row_off, table, nchunks, (uint32_t)chunk, (uint32_t)cspan, stride, cap,
-                       overflow);
-    hipError_t st = launch_scan(row_count, row_off, F.rows + 1, partials, stream);
-    if (st != hipSuccess) return st;
-    hipLaunchKernelGGL(k_rows_pass<true>, grid, dim3(64 * kRowWaves), dyn, stream, F, start, row_count,
-                       (const uint32_t*)row_off, table, nchunks, (uint32_t)chunk, (uint32_t)cspan, stride, cap,
-                       overflow);
-    return hipGetLastError();
-}
-
-static hipError_t launch_sort_runs(uint32_t n, const uint32_t* key, uint32_t* perm, uint32_t* permid, hipStream_t stream)
-{
-    if (n == 0) return hipSuccess;
-    if (n <= (1u << 26))
-        hipLaunchKernelGGL(k_sort_runs<uint32_t>, dim3(blocks_for(n)), dim3(kBlock), 0, stream, n, key, perm, permid);
-    else
-        hipLaunchKernelGGL(k_sort_runs<uint64_t>, dim3(blocks_for(n)), dim3(kBlock), 0, stream, n, key, perm, permid);
-    return hipGetLastError();
-}
-
-hipError_t launch_scatter_ranked(uint32_t n, const uint32_t* key, const uint32_t* rank, const uint32_t* start,
-                                 const uint32_t* id, uint32_t* perm, uint32_t* permid, hipStream_t stream)
-{
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_scatter_ranked, dim3(blocks_for(n)), dim3(kBlock), 0, stream, n, key, rank, start, id,
-                       perm, permid);
+    R.blocks = (F.rows + kRowWaves - 1) / kRowWaves;
+    R.stride = (uint32_t)max_cols + 1;
+    const dim3 grid(R.blocks + blocks_for(F.n));
+    const size_t dyn = sizeof(uint32_t) * kRowWaves * R.stride;
+    hipLaunchKernelGGL(k_scatter_ranked, grid, dim3(kBlock), dyn, stream, F, R, key, rank, start, id, perm, permid);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
-    return launch_sort_runs(n, key, perm, permid, stream);
+    R.off = nullptr;
+    if (F.rows > kRowsSum) {
+        if ((err = launch_scan(R.count, row_off, F.rows, partials, stream)) != hipSuccess) return err;
+        R.off = row_off;
+    }
+    if (F.n <= (1u << 26))
+        hipLaunchKernelGGL(k_sort_runs<uint32_t>, grid, dim3(kBlock), dyn, stream, F, R, key, start, perm, permid);
+    else
+        hipLaunchKernelGGL(k_sort_runs<uint64_t>, grid, dim3(kBlock), dyn, stream, F, R, key, start, perm, permid);
+    return hipGetLastError();
 }
 
 hipError_t launch_gather(Flocks F, const uint32_t* perm, const uint32_t* permid, const uint32_t* key,

@@ -118,8 +118,8 @@ typedef struct {
 /* Kernel ids for bs_get_timing. */
 enum {
     BS_K_PAIR = 0,       /* fused neighbour + integrate kernel (all modes) */
-    BS_K_SCAN = 1,       /* cell-count scan + block table */
-    BS_K_SCATTER = 2,    /* counting-sort scatter */
+    BS_K_SCAN = 1,       /* cell-count scan */
+    BS_K_SCATTER = 2,    /* counting-sort scatter, chunk table */
     BS_K_GATHER = 3,     /* in-cell rank + state gather */
     BS_K_OTHER = 4,
     BS_K_STEP = 5,       /* whole graph-replayed updates (BS_FLAG_GRAPH) */
