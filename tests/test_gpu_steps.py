@@ -96,3 +96,24 @@ def test_scan_sizes(cells):
         check(e, single(e, n, 1.0), f"{cells} cells per axis")
         e.step(1)
     e.close()
+
+
+@pytest.mark.parametrize("mode", [E.MODE_GRID_F64, E.MODE_GRID_MIXED])
+@pytest.mark.parametrize("n", [5, 1000, 13107, 16384, 32767, 32768])
+def test_small_flocks_run_in_small_chunks(mode, n):
+    # chunks of 6 boids, between 6 and 16, of 16 (their size never shows in the result)
+    F = max(1.0, (n / 16384.0) ** (1 / 3))
+    print(mode, n, flush=True)
+    st = flock(n, False, n).astype(np.float32)
+    a, b = (B.Engine(B.make_params(n, F, **RULES, mode=mode, flags=E.FLAG_DIGEST, fill=f)) for f in (0, 100))
+    for e in (a, b):
+        e.set_state(xyzv6=st)
+    for t in range(3):
+        for e in (a, b):
+            e.step(1)
+        check(a, single(a, n, F), f"n={n} update {t}")
+        assert a.grid()[0].chunk_boids == 64 * max(10, 100 * n // (64 * 2048)) // 100
+        assert np.array_equal(a.digest(), b.digest()), t
+        assert all(np.array_equal(x, y) for x, y in zip(a.state_f64(), b.state_f64())), t
+    a.close()
+    b.close()
