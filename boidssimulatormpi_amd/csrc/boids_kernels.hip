@@ -86,6 +86,69 @@ __global__ __launch_bounds__(kBlock) void k_allpairs_wave(DevParams P, St in, St
     out.x[i] = px; out.y[i] = py; out.z[i] = pz; out.vx[i] = vx; out.vy[i] = vy; out.vz[i] = vz;
 }
 
+// The same for small flocks: four waves per boid test the candidates, a quarter
+// of the batches each four at a time in flight, and leave each batch's
+// ballot in LDS; the first wave expands the ballots (lane b those of batch b,
+// hence at most 64 batches) into the list of ids and sums.  One update, one wave
+// per boid / this: float N = 256 6.5 / 5.9 us, 1000 10.3 / 6.6, 2048 15.6 / 10.2,
+// 4096 25.2 / 20.9; FP64 1024 11.3 / 7.8, 2048 15.9 / 13.4, 3000 22.8 / 21.2, 4096
+// 31.5 / 31.9 (in double the chip is full by then: the line lies at 3072).
+constexpr uint32_t kSmallFlock = 4096;
+
+template <typename R, typename St>
+__global__ __launch_bounds__(kBlock) void k_allpairs_small(DevParams P, St in, St out, R* forces, uint64_t* digest)
+{
+    __shared__ uint64_t ballots[kSmallFlock / 64];
+    __shared__ uint16_t list[kSmallFlock];
+    __shared__ typename OrderedSums<R>::Terms terms;
+    const uint32_t n = P.n, i = blockIdx.x;              // the grid has one workgroup per boid
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    R px = in.x[i], py = in.y[i], pz = in.z[i], vx = in.vx[i], vy = in.vy[i], vz = in.vz[i];
+    const R reach = reach_of(P, px, py, pz), F = (R)P.F, inv_F = (R)1 / F;
+    const uint32_t batches = (n + 63) / 64;              // <= 64
+    for (uint32_t b0 = wave; b0 < batches; b0 += 4 * kWaveOwners) {      // four batches' loads at once
+        R x[4], y[4], z[4];
+#pragma unroll
+        for (uint32_t t = 0; t < 4; ++t) {
+            const uint32_t at = min(64 * (b0 + t * kWaveOwners) + lane, n - 1);
+            x[t] = in.x[at]; y[t] = in.y[at]; z[t] = in.z[at];
+        }
+#pragma unroll
+        for (uint32_t t = 0; t < 4; ++t) {
+            const uint32_t b = b0 + t * kWaveOwners, j = 64 * b + lane;
+            const R s = near2(x[t] - px, y[t] - py, z[t] - pz, F, inv_F);
+            const uint64_t mask = __builtin_amdgcn_ballot_w64((j < n) & (j != i) & (s < reach));
+            if (lane == 0 && b < batches) ballots[b] = mask;
+        }
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    uint64_t mask = lane < batches ? ballots[lane] : 0;
+    const uint32_t mine = (uint32_t)__popcll(mask);
+    uint32_t incl = mine;
+#pragma unroll
+    for (uint32_t d = 1; d < 64; d <<= 1) {
+        const uint32_t t = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += t;
+    }
+    const uint32_t held = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    for (uint32_t at = incl - mine; mask; mask &= mask - 1)
+        list[at++] = (uint16_t)(64 * lane + (uint32_t)__builtin_ctzll(mask));
+    wave_lds_order();
+    const R vn = norm3(vx, vy, vz);
+    OrderedSums<R> S;
+    for (uint32_t h = 0; h < held; h += 64)
+        S.add(P, in, px, py, pz, vx, vy, vz, vn, lane, min(64u, held - h), h + lane < held ? (uint32_t)list[h + lane] : 0u,
+              terms, digest != nullptr);
+    if (digest) S.hash_sums();
+    const R dv[9] = {S.total(0), S.total(1), S.total(2), S.total(3), S.total(4),
+                     S.total(5), S.total(6), S.total(7), S.total(8)};
+    if (lane != 0) return;
+    finish_ordered(P, S, dv, i, px, py, pz, vx, vy, vz, forces, digest);
+    out.x[i] = px; out.y[i] = py; out.z[i] = pz; out.vx[i] = vx; out.vy[i] = vy; out.vz[i] = vz;
+}
+
 // ---------------------------------------------------------------------------
 // Grid build: cell hash + count, exclusive scan, scatter, in-cell rank +
 // gather.  Sorted order is (cell, boid id), independent of history.  Keys
@@ -508,22 +571,28 @@ __global__ __launch_bounds__(kBlock) void k_unpack_f32(uint32_t n, const float* 
 // ---------------------------------------------------------------------------
 static inline uint32_t blocks_for(uint32_t n) { return (n + kBlock - 1) / kBlock; }
 
+template <typename R, typename St>
+static hipError_t launch_allpairs(const DevParams& P, St in, St out, R* forces, uint64_t* digest, hipStream_t stream)
+{
+    if (P.n == 0) return hipSuccess;
+    if (P.n <= (sizeof(R) == 4 ? kSmallFlock : 3072))      // k_allpairs_small has the figures
+        hipLaunchKernelGGL((k_allpairs_small<R, St>), dim3(P.n), dim3(kBlock), 0, stream, P, in, out, forces, digest);
+    else
+        hipLaunchKernelGGL((k_allpairs_wave<R, St>), dim3((P.n + kWaveOwners - 1) / kWaveOwners), dim3(kBlock), 0,
+                           stream, P, in, out, forces, digest);
+    return hipGetLastError();
+}
+
 hipError_t launch_allpairs_f32ref(const DevParams& P, StateF32 in, StateF32 out, float* forces,
                                   uint64_t* digest, hipStream_t stream)
 {
-    if (P.n == 0) return hipSuccess;
-    hipLaunchKernelGGL((k_allpairs_wave<float, StateF32>), dim3((P.n + kWaveOwners - 1) / kWaveOwners),
-                       dim3(kBlock), 0, stream, P, in, out, forces, digest);
-    return hipGetLastError();
+    return launch_allpairs(P, in, out, forces, digest, stream);
 }
 
 hipError_t launch_allpairs_f64(const DevParams& P, StateF64 in, StateF64 out, double* forces,
                                uint64_t* digest, hipStream_t stream)
 {
-    if (P.n == 0) return hipSuccess;
-    hipLaunchKernelGGL((k_allpairs_wave<double, StateF64>), dim3((P.n + kWaveOwners - 1) / kWaveOwners),
-                       dim3(kBlock), 0, stream, P, in, out, forces, digest);
-    return hipGetLastError();
+    return launch_allpairs(P, in, out, forces, digest, stream);
 }
 
 hipError_t launch_hash_count(Flocks F, StateF64 st, uint32_t* key, uint32_t* rank, uint32_t* count,

@@ -27,10 +27,11 @@ def flock(n, far, seed):
 
 
 @pytest.mark.parametrize("mode", [E.MODE_ALLPAIRS_F32REF, E.MODE_ALLPAIRS_F64])
-@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 127, 128, 129, 1000])
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 127, 128, 129, 1000, 3072, 3073, 4095, 4096, 4097, 5003])
 @pytest.mark.parametrize("far", [False, True])
 def test_allpairs_equals_oracle(mode, n, far):
-    # one batch, several, and their remainders; lists that fill in the middle of the flock
+    # one batch, several, and their remainders, up to 3072 and 4096 boids and beyond; lists
+    # that fill in the middle of the flock
     print(mode, n, far, flush=True)
     f32 = mode == E.MODE_ALLPAIRS_F32REF
     st = flock(n, far, n)
