@@ -239,6 +239,17 @@ static int hip_fail(bs_engine* e, hipError_t st, const char* what)
     return fail(e, BS_E_HIP, std::string(what) + ": " + hipGetErrorString(st));
 }
 
+// A call makes its events, memory and launches on the engine's device; the
+// caller's current device comes back when it returns.
+struct OnDevice {
+    int callers = -1;
+    explicit OnDevice(const bs_engine* e)
+    {
+        if (hipGetDevice(&callers) != hipSuccess || callers == e->device || hipSetDevice(e->device) != hipSuccess) callers = -1;
+    }
+    ~OnDevice() { if (callers >= 0) (void)hipSetDevice(callers); }
+};
+
 #define HIP_TRY(e, expr)                                               \
     do {                                                               \
         hipError_t st_ = (expr);                                       \
@@ -1121,7 +1132,7 @@ static int transfer(bs_engine* e, const Span (&a)[2], char* dev, bool to_host, S
     std::atomic<int> error{(int)hipSuccess};
     auto carry = [&](unsigned w) {
         char* stage = loan.p + w * kPiece;
-        hipError_t st = hipSetDevice(e->device);
+        hipError_t st = w ? hipSetDevice(e->device) : hipSuccess;   // (a new thread starts on device 0)
         if (to_host)                                         // its share of the caller's pages
             for (const Span& s : a) {
                 const size_t share = (s.bytes / threads + 4095) & ~(size_t)4095, from = std::min(s.bytes, w * share);
@@ -1176,6 +1187,7 @@ extern "C" int bs_set_state_f64(bs_engine* e, const double* pos3, const double* 
     const uint32_t n = e->prm.n;
     if (n && (!pos3 || !vel3)) return fail(e, BS_E_ARG, "bs_set_state_f64: NULL array");
     if (is_f32(e->mode)) return fail(e, BS_E_STATE, "float-state mode: use bs_set_state_f32");
+    const OnDevice on(e);
     const StateF64 st = is_grid(e->mode) ? e->db : e->da;
     const Span a[2] = {{(char*)pos3, sizeof(double) * 3 * n}, {(char*)vel3, sizeof(double) * 3 * n}};
     StageLoan loan;
@@ -1190,6 +1202,7 @@ extern "C" int bs_set_state_f32(bs_engine* e, const float* xyzv6)
     if (!e) return BS_E_ARG;
     const uint32_t n = e->prm.n;
     if (n && !xyzv6) return fail(e, BS_E_ARG, "bs_set_state_f32: NULL array");
+    const OnDevice on(e);
     const Span a[2] = {{(char*)xyzv6, sizeof(float) * 6 * n}, {nullptr, 0}};
     StageLoan loan;
     int rc = transfer(e, a, (char*)e->tmp_pos, false, loan);
@@ -1235,6 +1248,7 @@ static int get_state(bs_engine* e, T* pos3, T* vel3, const char* what)
     const uint32_t n = e->prm.n;
     if (n && (!pos3 || !vel3)) return fail(e, BS_E_ARG, std::string(what) + ": NULL array");
     if (!e->has_state) return fail(e, BS_E_STATE, "no state: call bs_set_state_* first");
+    const OnDevice on(e);
     T* tmp = (T*)e->tmp_pos;
     const size_t bytes = sizeof(T) * 6 * n;
     StageLoan loan;
@@ -1273,6 +1287,7 @@ extern "C" int bs_get_forces_f64(bs_engine* e, double* f9)
     const size_t n9 = 9 * (size_t)e->prm.n;
     if (!e->forces) return fail(e, BS_E_STATE, "engine created without BS_FLAG_FORCES");
     if (n9 && !f9) return fail(e, BS_E_ARG, "bs_get_forces_f64: NULL array");
+    const OnDevice on(e);
     if (is_f32(e->mode)) {
         std::vector<float> tmp(n9);
         const Span a[2] = {{(char*)tmp.data(), sizeof(float) * n9}, {nullptr, 0}};
@@ -1293,6 +1308,7 @@ extern "C" int bs_get_forces_f32(bs_engine* e, float* f9)
     const size_t n9 = 9 * (size_t)e->prm.n;
     if (!e->forces) return fail(e, BS_E_STATE, "engine created without BS_FLAG_FORCES");
     if (n9 && !f9) return fail(e, BS_E_ARG, "bs_get_forces_f32: NULL array");
+    const OnDevice on(e);
     if (is_f32(e->mode)) {
         const Span a[2] = {{(char*)f9, sizeof(float) * n9}, {nullptr, 0}};
         StageLoan loan;
@@ -1392,6 +1408,7 @@ extern "C" int bs_step(bs_engine* e, uint32_t nsteps)
 {
     if (!e) return BS_E_ARG;
     if (!e->has_state) return fail(e, BS_E_STATE, "no state: call bs_set_state_* first");
+    const OnDevice on(e);
     if (is_grid(e->mode) && (e->prm.flags & BS_FLAG_GRAPH) && nsteps) {
         int rc = capture_step(e);
         if (rc) return rc;
@@ -1569,6 +1586,7 @@ static int metrics_impl(bs_engine* e, uint32_t flock, double eps, uint32_t min_s
     const double F = e->flocks.empty() ? e->prm.field : e->flock_field[flock];
     memset(out, 0, sizeof(*out));
     if (n == 0) return BS_OK;
+    const OnDevice on(e);
     // edge >= eps (links need only the 27 neighbouring cells); no more cells than
     // boids: eight per boid, as the static scratch is still priced, left most
     // searches for a third ring of 98 cells

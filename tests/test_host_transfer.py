@@ -1,0 +1,94 @@
+"""The engine's host code -- transfers, staging, devices -- over a stand-in for
+the HIP runtime (host_runtime.cpp: several devices in host memory, kernels do
+nothing, copies wait on their stream).  Each test runs in a process of its own,
+which loads the stand-in ahead of the engine."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+ROOT = os.path.abspath(os.path.join(os.path.dirname(__file__), ".."))
+
+PRELUDE = """
+import ctypes, sys
+import numpy as np
+rt = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)
+for name in ("rt_device_bytes", "rt_in_flight", "rt_calls", "rt_direct_bytes"):
+    getattr(rt, name).restype = ctypes.c_uint64
+import boidssimulatormpi_amd as B
+from boidssimulatormpi_amd import engine as E
+L = B.lib()
+RULES = dict(sep=(0.02, 0.75, 0.002), ali=(0.05, 0.75, 0.06), coh=(0.08, 0.75, 0.008), vmax=0.005, vmin=0.001)
+F64 = ctypes.POINTER(ctypes.c_double)
+
+def engine(n, device=0, mode=E.MODE_ALLPAIRS_F64, flags=E.FLAG_FORCES):
+    e = B.Engine(B.make_params(n, 1.0, **RULES, mode=mode, flags=flags, device=device))
+    assert rt.rt_calls(b"hipMalloc")               # the engine's calls end up in the stand-in
+    return e
+
+def state(n, seed=0):
+    g = np.random.default_rng(seed)
+    return g.random((n, 3)), g.random((n, 3))
+"""
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("rt") / "host_runtime.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-o", so, os.path.join(ROOT, "tests", "host_runtime.cpp")], check=True)
+    return so
+
+
+def drive(runtime, body):
+    r = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(body), runtime], cwd=ROOT, text=True,
+                       capture_output=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+# the staging's ways: one copy, several parts, pieces of several threads
+SIZES = (1000, 30000, 400000)
+
+
+def test_round_trip(runtime):
+    # (the stand-in's kernels do nothing: what comes back is what the upload left in the transfer buffer)
+    drive(runtime, f"""
+    for n in {SIZES[1:]}:
+        e = engine(n)
+        for seed in (1, 2):
+            p, v = state(n, seed)
+            e.set_state(pos=p, vel=v)
+            q, w = e.state_f64()
+            assert np.array_equal(p, q) and np.array_equal(v, w), n
+        assert not e.forces_f64().any()
+        e.close()
+    assert rt.rt_in_flight() == 0 and rt.rt_device_bytes(-1) == 0
+    """)
+
+
+@pytest.mark.parametrize("n", SIZES)
+def test_engines_on_several_devices(runtime, n):
+    # an engine works on its own device whatever the caller's is, which stays as it was
+    drive(runtime, f"""
+    n = {n}
+    engines = [engine(n, device=k) for k in range(3)]
+    for d in (3, 1):
+        rt.hipSetDevice(d)
+        for k, e in enumerate(engines):
+            p, v = state(n, k)
+            held = [rt.rt_device_bytes(j) for j in range(4)]
+            e.set_state(pos=p, vel=v)
+            e.step(2)
+            q, w = e.state_f64()
+            e.forces_f64()
+            e.metrics(0.02)
+            e.sync()
+            assert rt.rt_current() == d
+            assert [rt.rt_device_bytes(j) for j in range(4) if j != k] == [held[j] for j in range(4) if j != k]
+            assert n < 11000 or np.array_equal(p, q) and np.array_equal(v, w)
+    for e in engines:
+        e.close()
+    assert rt.rt_device_bytes(-1) == 0
+    """)
