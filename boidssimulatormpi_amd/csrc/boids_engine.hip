@@ -1019,15 +1019,16 @@ constexpr unsigned kStageThreads = 6;
 constexpr size_t kMapped = (size_t)1 << 19;
 static_assert(kStageThreads <= sizeof(((bs_engine*)0)->stage_ev) / sizeof(hipEvent_t), "an event per thread");
 
-// A call's hold on the staging it uses; `reader` is a stream that may still
-// be copying out of it when the call ends.
+// A call's hold on the staging it uses; `busy` is a stream whose work may still
+// read or write it when the call ends (from the first copy on, until the call
+// has waited for the last one -- so also where it fails in between).
 struct StageLoan {
     char* p = nullptr;
     size_t bytes = 0;
-    hipStream_t reader = nullptr;
+    hipStream_t busy = nullptr;
     ~StageLoan()
     {
-        if (reader) (void)hipStreamSynchronize(reader);
+        if (busy) (void)hipStreamSynchronize(busy);
         stage_back(p, bytes);
     }
 };
@@ -1045,6 +1046,7 @@ static bool lend_stage(bs_engine* e, size_t bytes, StageLoan& loan)
             return false;
         }
     loan.p = stage_take(want, &loan.bytes);
+    if (loan.p) loan.busy = e->stream;
     return loan.p != nullptr;
 }
 
@@ -1081,7 +1083,7 @@ static void copy_part(const Span* a, size_t at, char* stage, size_t bytes, bool 
 
 // Copies the two arrays (end to end at dev) to or from the device, after the
 // work queued on the engine's stream; returns once done, except that a copy to
-// the device may still be reading the staging (loan.reader).
+// the device may still be reading the staging (loan.busy).
 static int transfer(bs_engine* e, const Span (&a)[2], char* dev, bool to_host, StageLoan& loan)
 {
     const size_t total = a[0].bytes + a[1].bytes;
@@ -1113,10 +1115,10 @@ static int transfer(bs_engine* e, const Span (&a)[2], char* dev, bool to_host, S
             HIP_TRY(e, k + 1 < parts ? hipEventSynchronize(e->stage_ev[k]) : hipStreamSynchronize(e->stream));
             copy_part(a, at, loan.p + at, std::min(part, total - at), true);
         }
+        loan.busy = nullptr;
         return BS_OK;
     }
     if (direct) {
-        loan.reader = e->stream;
         for (size_t at = 0; at < total; at += kPart) {
             const size_t len = std::min(kPart, total - at);
             copy_part(a, at, loan.p + at, len, false);
@@ -1162,6 +1164,7 @@ static int transfer(bs_engine* e, const Span (&a)[2], char* dev, bool to_host, S
     carry(0);
     for (unsigned w = 0; w < started; ++w) helpers[w].join();
     HIP_TRY(e, (hipError_t)error.load());
+    loan.busy = nullptr;
     return BS_OK;
 }
 
@@ -1175,7 +1178,7 @@ static int settle_state(bs_engine* e, StateF64 st, StageLoan& loan)
         if (rc) return rc;
     }
     HIP_TRY(e, hipStreamSynchronize(e->stream));
-    loan.reader = nullptr;
+    loan.busy = nullptr;
     e->has_state = true;
     e->steps = 0;
     return BS_OK;
@@ -1215,7 +1218,7 @@ extern "C" int bs_set_state_f32(bs_engine* e, const float* xyzv6)
             HIP_TRY(e, launch_f32_hash(e->P, e->fa, e->key, e->rank, e->count, e->outside, e->stream));
         }
         HIP_TRY(e, hipStreamSynchronize(e->stream));
-        loan.reader = nullptr;
+        loan.busy = nullptr;
         e->has_state = true;
         e->steps = 0;
         return BS_OK;
@@ -1260,6 +1263,7 @@ static int get_state(bs_engine* e, T* pos3, T* vel3, const char* what)
         prefault((char*)pos3, bytes / 2);
         prefault((char*)vel3, bytes / 2);
         HIP_TRY(e, hipStreamSynchronize(e->stream));
+        loan.busy = nullptr;
         memcpy(pos3, out, bytes / 2);
         memcpy(vel3, out + 3 * (size_t)n, bytes / 2);
         return check_grid(e);

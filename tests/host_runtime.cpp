@@ -21,6 +21,7 @@
 namespace {
 constexpr int kDevices = 4;
 thread_local int current = 0;
+thread_local hipError_t last = hipSuccess;
 std::recursive_mutex mu;
 struct Mem { size_t bytes; int device; bool host; };
 std::map<char*, Mem> mem;
@@ -69,7 +70,7 @@ hipError_t give(void* p)
 }  // namespace
 
 #define LOCK std::lock_guard<std::recursive_mutex> lk(mu)
-#define MAY_FAIL(name) if (fails(name)) return hipErrorUnknown
+#define MAY_FAIL(name) if (fails(name)) return last = hipErrorUnknown
 
 // An allocation failure inside the engine's own calls, on the calling thread.
 void* operator new(size_t n)
@@ -117,7 +118,7 @@ uint64_t rt_in_flight(void)
 hipError_t hipSetDevice(int d) { LOCK; MAY_FAIL("hipSetDevice"); if (d < 0 || d >= kDevices) return hipErrorInvalidDevice; current = d; return hipSuccess; }
 hipError_t hipGetDevice(int* d) { *d = current; return hipSuccess; }
 hipError_t hipGetDeviceCount(int* n) { *n = kDevices; return hipSuccess; }
-hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipGetLastError(void) { const hipError_t e = last; last = hipSuccess; return e; }
 const char* hipGetErrorString(hipError_t e) { return e == hipErrorInvalidHandle ? "invalid handle" : e == hipErrorUnknown ? "made to fail" : "error"; }
 hipError_t hipMalloc(void** p, size_t n) { LOCK; MAY_FAIL("hipMalloc"); return take(p, n, false); }
 hipError_t hipFree(void* p) { LOCK; return give(p); }
@@ -205,6 +206,16 @@ hipError_t hipMemsetAsync(void* to, int v, size_t n, hipStream_t s)
     LOCK;
     ((Stream*)s)->ops.push_back({[=] { memset(to, v, n); }, (char*)to, nullptr});
     ++((Stream*)s)->queued;
+    return hipSuccess;
+}
+// (what a launch expands to: the stream goes through here)
+static thread_local hipStream_t launch_stream = nullptr;
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t s) { launch_stream = s; return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shared, hipStream_t* s)
+{
+    *grid = *block = dim3(1);
+    *shared = 0;
+    *s = launch_stream;
     return hipSuccess;
 }
 hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t s)

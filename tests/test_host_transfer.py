@@ -92,3 +92,34 @@ def test_engines_on_several_devices(runtime, n):
         e.close()
     assert rt.rt_device_bytes(-1) == 0
     """)
+
+
+@pytest.mark.parametrize("call", ["hipMemcpyAsync", "hipEventRecord", "hipEventSynchronize", "hipStreamSynchronize",
+                                  "hipLaunchKernel"])
+def test_failed_transfers_leave_no_copy_behind(runtime, call):
+    # whichever call of a transfer fails, nothing still reads or writes the staging once it is lent again
+    drive(runtime, f"""
+    for n in {SIZES}:
+        e = engine(n)
+        p, v = state(n)
+        failed = 0
+        for op in (lambda: e.set_state(pos=p, vel=v), e.state_f64, e.forces_f64, e.state_f32):
+            e.set_state(pos=p, vel=v)
+            for k in range(1, 14):
+                rt.rt_fail(b"{call}", k)
+                try:
+                    op()
+                except B.EngineError as err:
+                    failed += 1
+                    assert "made to fail" in str(err)
+                rt.rt_fail(b"{call}", 0)
+                rt.hipGetLastError()
+                assert rt.rt_in_flight() == 0, (n, k)
+        assert failed or "Event" in "{call}" and n == 1000
+        e.set_state(pos=p, vel=v)
+        if n > 11000:
+            q, w = e.state_f64()
+            assert np.array_equal(p, q) and np.array_equal(v, w)
+        e.close()
+    assert rt.rt_device_bytes(-1) == 0
+    """)
