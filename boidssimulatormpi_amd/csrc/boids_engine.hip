@@ -50,7 +50,6 @@ static_assert(BS_MIXED_CHUNK_SPAN >= 1 && BS_MIXED_CHUNK_SPAN <= boids::kChunkSp
 #include <map>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -1157,8 +1156,8 @@ static int transfer(bs_engine* e, const Span (&a)[2], char* dev, bool to_host, S
         try {
             helpers[started] = std::thread(carry, w);
             ++started;
-        } catch (const std::system_error&) {
-            break;                                           // no more threads: the started ones carry it all
+        } catch (...) {
+            break;                                           // no thread or no memory for one: the started ones carry it all
         }
     }
     carry(0);

@@ -31,7 +31,9 @@ struct Event { int device; Stream* on; uint64_t at; };
 std::map<std::string, int> countdown;
 std::map<std::string, uint64_t> calls;
 uint64_t direct = 0;                                   // bytes copied from the device to memory outside hipHostMalloc's
-thread_local int news_left = -1;                       // operator new fails on this thread when it reaches 0
+thread_local int news_left = 0, inside = 0;            // operator new fails on this thread when news_left comes
+                                                       // down to 0 (the stand-in's own calls do not count)
+struct Inside { Inside() { ++inside; } ~Inside() { --inside; } };
 
 bool fails(const char* name)
 {
@@ -69,13 +71,13 @@ hipError_t give(void* p)
 }
 }  // namespace
 
-#define LOCK std::lock_guard<std::recursive_mutex> lk(mu)
+#define LOCK std::lock_guard<std::recursive_mutex> lk(mu); Inside in
 #define MAY_FAIL(name) if (fails(name)) return last = hipErrorUnknown
 
 // An allocation failure inside the engine's own calls, on the calling thread.
 void* operator new(size_t n)
 {
-    if (news_left > 0 && --news_left == 0) throw std::bad_alloc();
+    if (!inside && news_left > 0 && --news_left == 0) throw std::bad_alloc();
     void* p = malloc(n ? n : 1);
     if (!p) throw std::bad_alloc();
     return p;

@@ -123,3 +123,25 @@ def test_failed_transfers_leave_no_copy_behind(runtime, call):
         e.close()
     assert rt.rt_device_bytes(-1) == 0
     """)
+
+
+def test_transfers_without_memory_for_their_threads(runtime):
+    # a large transfer whose helper threads cannot be made is carried by those that could, or by the caller
+    drive(runtime, f"""
+    n = {SIZES[2]}
+    e = engine(n)
+    p, v = state(n)
+    q, w = np.empty_like(p), np.empty_like(v)
+    at = [a.ctypes.data_as(F64) for a in (p, v, q, w)]
+    e.set_state(pos=v, vel=p)
+    for k in range(1, 7):
+        rt.rt_fail_new(k)
+        assert L.bs_set_state_f64(e._h, at[0], at[1]) == 0
+        rt.rt_fail_new(k)
+        assert L.bs_get_state_f64(e._h, at[2], at[3]) == 0
+        rt.rt_fail_new(0)
+        assert np.array_equal(p, q) and np.array_equal(v, w)
+        p += 1.0
+        v -= 1.0
+    e.close()
+    """)
