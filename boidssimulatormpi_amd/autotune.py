@@ -29,7 +29,7 @@ CACHE_PATH = os.environ.get("BOIDS_TUNING_CACHE") or os.path.join(
 
 BLOCKS = (64, 128, 256)
 TILES = (5, 6, 9, 12)       # LDS candidates staged per thread and pass
-FILLS = (60, 80, 100)       # chunk fill target, percent of the workgroup
+FILLS = (0, 60, 80, 100)    # chunk size limit, percent of the workgroup (0: the engine's own, down to 10)
 CELL_SCALES = (1.0, 0.85)   # cells per axis relative to the automatic choice
 
 

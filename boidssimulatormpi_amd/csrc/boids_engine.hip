@@ -193,7 +193,7 @@ struct bs_engine {
     int cspan = kChunkSpanMax;         // most x columns a neighbour-kernel chunk covers
     int nb = 64;                       // neighbour-kernel workgroup size
     int tile = 12;                     // LDS tile depth (candidates per thread and pass)
-    int fill = 100;                    // chunk size target, percent of nb
+    int fill = 100;                    // chunk size limit, percent of nb
     uint32_t chunk = 256;              // boids per chunk at most (fill% of nb)
     bool batch = false;
     // one captured step (BS_FLAG_GRAPH)
@@ -726,25 +726,23 @@ static int create_engine(const bs_params* fp, uint32_t count, bool batch, bs_eng
             return fail(nullptr, BS_E_ARG, "block must be 0, 64, 128 or 256");
         }
         if (p->tile != 0 && p->tile != 5 && p->tile != 6 && p->tile != 9 && p->tile != 12) { release(e); return fail(nullptr, BS_E_ARG, "tile must be 0, 5, 6, 9 or 12"); }
-        if (p->fill != 0 && (p->fill < 25 || p->fill > 100)) { release(e); return fail(nullptr, BS_E_ARG, "fill must be 0 or 25..100"); }
+        if (p->fill != 0 && (p->fill < 10 || p->fill > 100)) { release(e); return fail(nullptr, BS_E_ARG, "fill must be 0 or 10..100"); }
         e->tile = p->tile ? p->tile : (p->mode == BS_MODE_GRID_MIXED ? BS_MIXED_TILE : BS_F64_TILE);
         // Automatic fill: full chunks, unless that leaves fewer than ~2048
         // of them (8 workgroups per CU) -- a small flock then runs in
         // smaller chunks, more workgroups in flight, each with a shorter chain
-        // (down to 10 %).  An update, FP64, uniform / n / 256 blobs, by fill:
+        // (down to 10 %, so a flock below 13108 boids makes fewer than 2048).
+        // An update, FP64, uniform / n / 256 blobs, by fill:
         //   n = 4096:  25 62 / 132 us, 16 58 / 118, 10 57 / 115, 7 60 / 118
         //   n = 16384: 25 64 / 183, 16 61 / 164, 12 63 / 158, 7 77 / 184
         //   n = 32768: 50 82 / 209, 25 77 / 180, 13 89 / 202
-        // (mixed alike).  `fill`, as bs_get_info gives it, stays in the range
-        // that bs_params takes.
-        uint64_t percent = 0;
+        // (mixed alike).
         {
             uint64_t nsum = 0;
             for (uint32_t k = 0; k < count; ++k) nsum += fp[k].n;
             const int nb_auto = p->block ? p->block : 64;
             const uint64_t want = 100 * nsum / ((uint64_t)nb_auto * 2048);
-            percent = p->fill ? p->fill : std::max<uint64_t>(10, std::min<uint64_t>(100, want));
-            e->fill = (int)std::max<uint64_t>(25, percent);
+            e->fill = p->fill ? p->fill : (int)std::max<uint64_t>(10, std::min<uint64_t>(100, want));
         }
         uint64_t cells = 0, rows = 0;
         bool coarse = false;
@@ -792,7 +790,7 @@ static int create_engine(const bs_params* fp, uint32_t count, bool batch, bs_eng
         // smaller LDS footprint more workgroups fit a CU (measured faster
         // than 128 for long rows too).
         e->nb = p->block ? p->block : 64;
-        e->chunk = std::max(1u, (uint32_t)percent * (uint32_t)e->nb / 100u);
+        e->chunk = (uint32_t)(e->fill * e->nb / 100);
         if (e->mode != BS_MODE_ALLPAIRS_F64) {
             if (cells + 1 > 0x7fffffffull) { release(e); return fail(nullptr, BS_E_ARG, "too many grid cells over all flocks"); }
             uint32_t base = 0;

@@ -98,8 +98,8 @@ typedef struct {
     int32_t tile;                /* grid modes: LDS tile depth, candidates staged per thread and pass:
                                   * 5, 6, 9 or 12; 0 = automatic (5) */
     int32_t fill;                /* grid modes: most boids per chunk, percent of the workgroup size
-                                  * (25..100); 0 = automatic (100, less for small flocks: about 2048
-                                  * chunks at least) */
+                                  * (10..100); 0 = automatic (100; less for small flocks, down to 10, for
+                                  * about 2048 chunks) */
 } bs_params;
 
 /* Read-only facts about a created engine. */
@@ -111,7 +111,7 @@ typedef struct {
     uint64_t steps;              /* updates done since the last set_state/init */
     int32_t block;               /* neighbour-kernel workgroup size (grid modes), else 0 */
     int32_t tile;                /* LDS tile depth (grid modes), else 0 */
-    int32_t fill;                /* chunk size limit in percent of block (grid modes), else 0 */
+    int32_t fill;                /* chunk size limit in use, in percent of block (grid modes), else 0 */
     int32_t reserved;
 } bs_info;
 

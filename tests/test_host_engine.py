@@ -1,4 +1,4 @@
-"""The engine's host code -- transfers, staging, devices -- over a stand-in for
+"""The engine's host code -- transfers, staging, devices, chunk sizes -- over a stand-in for
 the HIP runtime (host_runtime.cpp: several devices in host memory, kernels do
 nothing, copies wait on their stream).  Each test runs in a process of its own,
 which loads the stand-in ahead of the engine."""
@@ -144,4 +144,37 @@ def test_transfers_without_memory_for_their_threads(runtime):
         p += 1.0
         v -= 1.0
     e.close()
+    """)
+
+
+@pytest.mark.parametrize("mode", [2, 3])
+def test_chunk_size_as_reported(runtime, mode):
+    # bs_info.fill is the chunk size in use and, passed back, gives the same engine
+    drive(runtime, f"""
+    from boidssimulatormpi_amd import autotune as T
+
+    def grid(n, block, fill):
+        F = max(1.0, (n / 16384.0) ** (1 / 3))
+        e = B.Engine(B.make_params(n, F, **RULES, mode={mode}, block=block, fill=fill))
+        assert e.info().mode == {mode}
+        e.set_state(xyzv6=np.zeros((n, 6), np.float32))
+        out = e.info().fill, e.grid()[0].chunk_boids
+        e.close()
+        return out
+    for block in (0, 64, 128, 256):
+        for n in (27, 1000, 13107, 16384, 20000, 32767, 32768, 50021, 131072, 600000):
+            fill, boids = grid(n, block, 0)
+            assert 10 <= fill <= 100 and boids == fill * (block or 64) // 100, (block, n)
+            assert grid(n, block, fill) == (fill, boids)
+        for fill in (10, 11, 24, 25, 60, 100):
+            assert grid(3000, block, fill) == (fill, fill * (block or 64) // 100)
+    for fill in (-1, 1, 9, 101):
+        try:
+            grid(3000, 0, fill)
+        except B.EngineError as err:
+            assert "10..100" in str(err)
+        else:
+            assert False, fill
+    # the tuner times the engine's own choice too
+    assert any(ps[0].fill == 0 for _, ps in T.candidates(B.make_params(3000, 1.0, **RULES, mode={mode})))
     """)
