@@ -261,15 +261,9 @@ void k_f32_grid_wave(DevParams P, StateF32 in, StateF32 out, const float4* __res
         for (uint32_t r = 0; r < R; ++r) hb[64 * r + lane] = k[r];
     };
 
-    // Windows of ascending ids: all of them at once unless more are in reach
-    // than the list holds; then narrower ones (one id never overflows it).
-    for (uint32_t lo = 0, width = P.n; lo < P.n;) {
-        const uint32_t H = collect(lo, width);
-        if (H > kF32HitCap) {
-            const uint32_t w = (uint32_t)((uint64_t)width * (kF32HitCap * 3 / 4) / H);
-            width = max(1u, min(w, width / 2));
-            continue;
-        }
+    for (IdWindows ids(P.n, kF32HitCap); ids.more();) {
+        const uint32_t H = collect(ids.lo, ids.width);
+        if (!ids.take(H)) continue;
         wave_lds_order();
         if (H <= 64) {
             sorted(std::integral_constant<uint32_t, 1>{}, H);
@@ -298,7 +292,6 @@ void k_f32_grid_wave(DevParams P, StateF32 in, StateF32 out, const float4* __res
         for (uint32_t h0 = 0; h0 < H; h0 += 64)        // (3)
             S.add(P, in, px, py, pz, vx, vy, vz, vn, lane, min(64u, H - h0), h0 + lane < H ? hb[h0 + lane] : 0u, terms,
                   digest != nullptr);
-        lo += min(width, P.n - lo);
     }
 
     if (digest) S.hash_sums();

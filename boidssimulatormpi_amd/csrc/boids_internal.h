@@ -159,6 +159,38 @@ hipError_t launch_nbr_mixed(Flocks F, int nb, int tile, int max_cols, StateF64 i
                             uint32_t* count, double* forces, uint64_t* digest, uint32_t* recheck,
                             hipStream_t stream);
 hipError_t launch_copy(const void* src, void* dst, uint64_t bytes, hipStream_t stream);
+// The windows of ascending ids in which an owner of the float grid takes its
+// boids: all of them at once unless more are in reach than its list of `cap`
+// holds; then narrower ones, each sized from what the last one held.  Every
+// window is a pass over all candidates, so few of them count: one that
+// overflows narrows to what would fill 3/4 of the list, one that fills less
+// than a quarter widens fourfold (ids in clumps: the gaps before, between and
+// behind them take a logarithmic number), and the rest goes at once when it
+// fits.  Kept at the width first found, ids 2^19 .. 2^19 + 4000 of 2^20 took 671
+// passes, 24 this way (the update 37.1 ms, 4.8 now).  One id never overflows the list, so every pass ends in
+// progress.
+struct IdWindows {
+    uint32_t n, cap, lo = 0, width, left = ~0u;       // ids [lo, lo + width) next; boids in reach at lo or above
+    __host__ __device__ IdWindows(uint32_t n_, uint32_t cap_) : n(n_), cap(cap_), width(n_) {}
+    __host__ __device__ bool more() const { return left != 0 && lo < n; }
+    // `found` boids in the window: true if they fit (the window is done)
+    __host__ __device__ bool take(uint32_t found)
+    {
+        if (left == ~0u) left = found;                 // (the first window is all ids)
+        if (found > cap) {
+            const uint32_t w = (uint32_t)((uint64_t)width * (cap * 3 / 4) / found), half = width / 2;
+            width = w < half ? w : half;
+            if (width == 0) width = 1;
+            return false;
+        }
+        left -= found;
+        lo = width < n - lo ? lo + width : n;
+        if (left <= cap) width = n;
+        else if (found < cap / 4) width = 4 * width < n ? 4 * width : n;     // (n <= 2^28)
+        return true;
+    }
+};
+
 // Reference-faithful float grid (boids_f32grid.hip): cell keys, arrival ranks
 // and counts of a state from outside; the cell list from them (start, records);
 // the step from it (id order in, id order out), which leaves keys, ranks and

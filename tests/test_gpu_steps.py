@@ -118,3 +118,32 @@ def test_small_flocks_run_in_small_chunks(mode, n):
         assert all(np.array_equal(x, y) for x, y in zip(a.state_f64(), b.state_f64())), t
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("spread", ["first", "middle", "two clumps", "clump and dust"])
+def test_float_grid_crowds_of_neighbouring_ids(spread):
+    # more boids within reach than an owner's list holds, their ids side by side: several windows of ids
+    n, m = 9001, 2600
+    print(spread, flush=True)
+    g = np.random.default_rng(m)
+    ids = {"first": np.arange(m), "middle": np.arange(n // 2, n // 2 + m),
+           "two clumps": np.r_[1000: 1000 + m // 2, 7000: 7000 + m // 2],
+           "clump and dust": np.r_[5000: 5000 + m // 2, g.choice(5000, m // 2, replace=False)]}[spread]
+    st = flock(n, False, n).astype(np.float32)
+    st[::3, :3] = g.random((len(st[::3]), 3))              # (no other crowd)
+    st[ids, :3] = 0.4 + 0.01 * g.random((m, 3))
+    flags = E.FLAG_DIGEST | E.FLAG_FORCES
+    a = B.Engine(B.make_params(n, 1.0, **RULES, mode=E.MODE_ALLPAIRS_F32REF, flags=flags))
+    b = B.Engine(B.make_params(n, 1.0, **RULES, mode=E.MODE_GRID_F32REF, flags=flags))
+    assert b.info().mode == E.MODE_GRID_F32REF
+    for e in (a, b):
+        e.set_state(xyzv6=st)
+    for t in range(2):
+        for e in (a, b):
+            e.step(1)
+        assert t or ((a.digest()[ids, 0] >> 42) > 1024).all()          # alignment has no view cone here
+        assert np.array_equal(a.digest(), b.digest()), t
+        assert np.array_equal(a.forces_f32(), b.forces_f32()), t
+        assert all(np.array_equal(x, y) for x, y in zip(a.state_f32(), b.state_f32())), t
+    a.close()
+    b.close()
