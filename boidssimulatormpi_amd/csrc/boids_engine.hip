@@ -821,9 +821,15 @@ static int create_engine(const bs_params* fp, uint32_t count, bool batch, bs_eng
             e->P.G = G;
             // Half cells: the sphere around an owner then touches cells that hold a
             // third of the boids of the 27 whole ones.  Where eight times the cells
-            // would outgrow the boids (8 counters each) or 32 bits, whole ones.
+            // would outgrow the boids (8 counters each), whole ones.
+            // Whole ones also above 2^18 boids, where the records (16 bytes each)
+            // outgrow an XCD's 4 MB of L2: owners come in id order, so every row of a
+            // window is then read from beyond it, and half cells have 25 rows to 9.  An
+            // update, uniform / 64 blobs, half / whole cells: N = 2^18 497 / 511 and
+            // 1108 / 1182 us, 2^19 1277 / 1172 and 3428 / 3532, 2^20 2978 / 2675 and
+            // 8592 / 8826, 2^21 6586 / 5871 and 19311 / 19719.
             const uint64_t half = 8ull * G * G * G;
-            e->P.sx = half < (1ull << 31) && half <= std::max<uint64_t>(8ull * e->prm.n, 1u << 15) ? 2 : 1;
+            e->P.sx = e->prm.n <= (1u << 18) && half <= std::max<uint64_t>(8ull * e->prm.n, 1u << 15) ? 2 : 1;
             e->P.inv_edge = G / p->field;
             e->ncell1 = (uint32_t)((uint64_t)G * G * G * (e->P.sx == 2 ? 8 : 1) + 1);
         }

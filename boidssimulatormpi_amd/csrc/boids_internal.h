@@ -167,8 +167,8 @@ hipError_t launch_copy(const void* src, void* dst, uint64_t bytes, hipStream_t s
 // than a quarter widens fourfold (ids in clumps: the gaps before, between and
 // behind them take a logarithmic number), and the rest goes at once when it
 // fits.  Kept at the width first found, ids 2^19 .. 2^19 + 4000 of 2^20 took 671
-// passes, 24 this way (the update 37.1 ms, 4.8 now).  One id never overflows the list, so every pass ends in
-// progress.
+// passes (an update 37.1 ms), this way 24 (4.8 ms).  One id never overflows the
+// list, so every pass ends in progress.
 struct IdWindows {
     uint32_t n, cap, lo = 0, width, left = ~0u;       // ids [lo, lo + width) next; boids in reach at lo or above
     __host__ __device__ IdWindows(uint32_t n_, uint32_t cap_) : n(n_), cap(cap_), width(n_) {}

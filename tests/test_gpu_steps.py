@@ -147,3 +147,21 @@ def test_float_grid_crowds_of_neighbouring_ids(spread):
         assert all(np.array_equal(x, y) for x, y in zip(a.state_f32(), b.state_f32())), t
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("n", [1 << 18, (1 << 18) + 1])
+def test_float_grid_at_the_largest_half_cells(n):
+    # half cells up to 2^18 boids, whole ones beyond
+    print(n, flush=True)
+    F = (n / 16384.0) ** (1 / 3)
+    st = B.generate_init(E.INIT_CLUSTERED, n, F, 0.005, 0.001, seed=3)
+    a = B.Engine(B.make_params(n, F, **RULES, mode=E.MODE_ALLPAIRS_F32REF, flags=E.FLAG_DIGEST))
+    b = B.Engine(B.make_params(n, F, **RULES, mode=E.MODE_GRID_F32REF, flags=E.FLAG_DIGEST))
+    assert b.info().mode == E.MODE_GRID_F32REF
+    for e in (a, b):
+        e.set_state(xyzv6=st)
+        e.step(1)
+    assert np.array_equal(a.digest(), b.digest())
+    assert all(np.array_equal(x, y) for x, y in zip(a.state_f32(), b.state_f32()))
+    a.close()
+    b.close()
