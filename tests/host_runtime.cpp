@@ -30,7 +30,7 @@ struct Stream { int device; std::list<Op> ops; uint64_t done = 0, queued = 0; };
 struct Event { int device; Stream* on; uint64_t at; };
 std::map<std::string, int> countdown;
 std::map<std::string, uint64_t> calls;
-uint64_t direct = 0;                                   // bytes copied from the device to memory outside hipHostMalloc's
+std::map<char*, uint64_t> copied;                      // bytes that copies wrote into each block
 thread_local int news_left = 0, inside = 0;            // operator new fails on this thread when news_left comes
                                                        // down to 0 (the stand-in's own calls do not count)
 struct Inside { Inside() { ++inside; } ~Inside() { --inside; } };
@@ -66,6 +66,7 @@ hipError_t take(void** p, size_t bytes, bool host)
 hipError_t give(void* p)
 {
     if (p && !mem.erase((char*)p)) return hipErrorInvalidValue;
+    copied.erase((char*)p);
     free(p);
     return hipSuccess;
 }
@@ -101,7 +102,8 @@ uint64_t rt_device_bytes(int device)
 }
 // copies in flight that write or read memory from hipHostMalloc
 uint64_t rt_in_flight(void);
-uint64_t rt_direct_bytes(void) { LOCK; return direct; }
+// bytes that copies have written into the block at p
+uint64_t rt_copied_to(const void* p) { LOCK; return copied[(char*)p]; }
 
 static std::list<Stream*> streams;
 uint64_t rt_in_flight(void)
@@ -190,7 +192,6 @@ hipError_t hipMemcpyAsync(void* to, const void* from, size_t n, hipMemcpyKind ki
     if (kind == hipMemcpyDeviceToHost && b == mem.end()) {      // pageable memory: the runtime waits for it
         run((Stream*)s, ((Stream*)s)->queued);
         memcpy(to, from, n);
-        direct += n;
         return hipSuccess;
     }
     if (kind == hipMemcpyHostToDevice && block_of(from) == mem.end()) {
@@ -198,6 +199,8 @@ hipError_t hipMemcpyAsync(void* to, const void* from, size_t n, hipMemcpyKind ki
         memcpy(to, from, n);
         return hipSuccess;
     }
+    if (b == mem.end()) return hipErrorInvalidValue;
+    copied[b->first] += n;
     ((Stream*)s)->ops.push_back({[=] { memcpy(to, from, n); }, (char*)to, (char*)from});
     ++((Stream*)s)->queued;
     return hipSuccess;

@@ -3,6 +3,8 @@ changes its way: written by the kernel into pinned staging, copied through it
 in one or several parts, and cut into
 pieces that several threads carry (ragged last pieces, both arrays of a pair in
 one piece)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -52,3 +54,33 @@ def test_forces_agree_between_types(n):
         f64, f32 = e.forces_f64(), e.forces_f32()
         assert f64.any() and np.array_equal(f32, f64.astype(np.float32))
         e.close()
+
+
+@pytest.mark.parametrize("n", [1000, 8000, 21845, 21846, 130000, 400000])
+def test_outputs_into_pinned_memory(n):
+    # staged (two arrays up to 1 MiB) and straight; one array of a pair pinned, the other not
+    hip = ctypes.CDLL("libamdhip64.so")
+    f64 = ctypes.POINTER(ctypes.c_double)
+    F = max(1.0, (n / 16384.0) ** (1 / 3))
+    g = np.random.default_rng(n)
+    pos, vel = F * 0.999 * g.random((n, 3)), 1e-3 * g.standard_normal((n, 3))
+    print(n, flush=True)
+    for mode in (E.MODE_ALLPAIRS_F64, E.MODE_GRID_F64):
+        e = B.Engine(B.make_params(n, F, mode=mode, flags=E.FLAG_FORCES))
+        e.set_state(pos=pos, vel=vel)
+        p = ctypes.c_void_p()
+        assert hip.hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(72 * n), 0) == 0
+        pin = np.frombuffer((ctypes.c_char * (72 * n)).from_address(p.value), np.float64)
+        out = np.empty(9 * n)
+        for a, b in ((pin[:3 * n], pin[3 * n:6 * n]), (pin[:3 * n], out[:3 * n]), (out[:3 * n], pin[:3 * n])):
+            pin[:] = out[:] = np.nan
+            assert B.lib().bs_get_state_f64(e._h, a.ctypes.data_as(f64), b.ctypes.data_as(f64)) == 0
+            assert np.array_equal(a, pos.ravel()) and np.array_equal(b, vel.ravel())
+        if mode == E.MODE_GRID_F64:
+            e.step(1)
+        pin[:] = np.nan
+        assert B.lib().bs_get_forces_f64(e._h, pin.ctypes.data_as(f64)) == 0
+        assert np.array_equal(pin, e.forces_f64().ravel())
+        e.close()
+        del pin
+        assert hip.hipHostFree(p) == 0
