@@ -1006,16 +1006,20 @@ static int grid_sort_into_a(bs_engine* e)
 // How states and forces go in and out (24 bytes a boid in, 48 out; "before" is
 // the runtime's copy from or to the caller's pageable memory, one per array):
 //   up to kDirect: through the staging in parts, one part copied on the host
-//     while the next is under way (in: 10^4 boids 137 -> 60 us, 130000 boids 608
-//     -> 190 us; out, after queued updates: 14000 boids 101 -> 82 us, 130000
-//     402 -> 252 us);
+//     while the next is under way.  In, parts of kInPart (10^4 boids 137 -> 60 us,
+//     130000 boids 608 -> 190 us).  Out, one part up to 2 kOutPart and then equal
+//     ones of about kOutPart, 6 at most: a part of its own costs about 12 us, the
+//     copy on the host it hides about 40 us a MB (FP64 states after an update:
+//     16384 boids 193 us before, 163 in parts of 256 KB, 124 this way; 50021 321,
+//     270, 237; 116000 528, 384, 379);
 //   above it: in pieces of kPiece that up to kStageThreads threads carry, each
 //     through a piece of the staging of its own, so the copies to and from
 //     the caller's pages (a few GB/s a thread, page faults included) run
 //     beside one another and the DMA (2^20 boids: in 17.5 -> 1.0 ms, out 5.4
 //     -> 1.6 ms; below it starting the threads costs more than they save:
 //     130000 boids out 289 us).
-constexpr size_t kPiece = (size_t)2 << 20, kPart = (size_t)1 << 18, kDirect = (size_t)8 << 20;
+constexpr size_t kPiece = (size_t)2 << 20, kDirect = (size_t)8 << 20;
+constexpr size_t kInPart = (size_t)1 << 18, kOutPart = (size_t)1 << 20;
 constexpr unsigned kStageThreads = 6;
 // States up to this size are written to the staging by the kernel that puts
 // them in order (consecutive words), without a copy after it.
@@ -1127,7 +1131,8 @@ static int transfer(bs_engine* e, const Span (&a)[2], char* dev, bool to_host, S
     }
     if (direct && to_host) {
         // in parts: one leaves the staging while the next arrives
-        const size_t part = total <= 2 * kPart ? total : std::max(kPart, (total / kStageThreads + 4095) & ~(size_t)4095);
+        const size_t want = total <= 2 * kOutPart ? 1 : std::min<size_t>(kStageThreads, (total + kOutPart - 1) / kOutPart);
+        const size_t part = ((total + want - 1) / want + 4095) & ~(size_t)4095;
         const unsigned parts = (unsigned)((total + part - 1) / part);
         for (unsigned k = 0; k < parts; ++k) {
             const size_t at = k * part, len = std::min(part, total - at);
@@ -1144,8 +1149,8 @@ static int transfer(bs_engine* e, const Span (&a)[2], char* dev, bool to_host, S
         return BS_OK;
     }
     if (direct) {
-        for (size_t at = 0; at < total; at += kPart) {
-            const size_t len = std::min(kPart, total - at);
+        for (size_t at = 0; at < total; at += kInPart) {
+            const size_t len = std::min(kInPart, total - at);
             copy_part(a, at, loan.p + at, len, false);
             HIP_TRY(e, hipMemcpyAsync(dev + at, loan.p + at, len, hipMemcpyHostToDevice, e->stream));
         }

@@ -220,3 +220,17 @@ def test_outputs_in_memory_the_runtime_knows(runtime, n):
             assert free(ctypes.c_void_p(b)) == 0
     e.close()
     """)
+
+
+@pytest.mark.parametrize("n,parts", [(1000, 1), (16384, 1), (29127, 1), (29128, 3), (50021, 4), (116508, 6)])
+def test_outputs_leave_in_few_parts(runtime, n, parts):
+    # forces (72 bytes a boid) into pageable memory: up to 2 MiB one copy, then parts of about 1 MiB, 6 at most;
+    # parts of 256 KiB took 1.5 times as long as the runtime's own copy (16384 boids 80 -> 116 us, one copy 68)
+    drive(runtime, f"""
+    e = engine({n})
+    e.forces_f64()
+    before = rt.rt_calls(b"hipMemcpyAsync")
+    e.forces_f64()
+    assert rt.rt_calls(b"hipMemcpyAsync") - before == {parts}, rt.rt_calls(b"hipMemcpyAsync") - before
+    e.close()
+    """)
