@@ -203,6 +203,23 @@ hipError_t launch_f32_grid_sort(const DevParams& P, StateF32 st, const uint32_t*
 hipError_t launch_f32_grid_step(const DevParams& P, StateF32 in, StateF32 out, const float4* rec, uint32_t* key,
                                 uint32_t* rank, const uint32_t* start, uint32_t* count, uint32_t* outside,
                                 float* forces, uint64_t* digest, hipStream_t stream);
+// Cells x0..x1 of a row of G, which wrap around the field (-G < x0 <= x1 < 2 G,
+// fewer than G of them): part 0 are those inside [0, G), part 1 the ones that
+// wrap, as cells a..z of the row (a > z: none).
+__host__ __device__ inline void wrapped_run(int x0, int x1, int G, int part, int* a, int* z)
+{
+    if (part == 0) {
+        *a = x0 < 0 ? 0 : x0;
+        *z = x1 < G ? x1 : G - 1;
+    } else if (x0 < 0) {
+        *a = x0 + G;
+        *z = (x1 < 0 ? x1 : -1) + G;
+    } else {
+        *a = x0 < G ? 0 : x0 - G;
+        *z = x1 - G;
+    }
+}
+
 // flock metrics (boids_metrics.hip)
 size_t metrics_workspace_bytes(uint32_t n, int G);
 // What the static scratch is priced at: 64 bytes per boid and 8 per cell of a

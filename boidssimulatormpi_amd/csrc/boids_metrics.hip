@@ -195,9 +195,9 @@ __global__ __launch_bounds__(kBlock) void k_m_near(MGrid g, const uint32_t* __re
             const uint32_t rw = (uint32_t)G * ((uint32_t)y + (uint32_t)G * (uint32_t)z);
             auto run = [&](int x0, int x1) {                      // cells x0..x1 of the row, unwrapped, x1 - x0 < G
                 for (int part = 0; part < 2; ++part) {
-                    const int a = part == 0 ? max(x0, 0) : (x0 < 0 ? x0 + G : 0);
-                    const int z1 = part == 0 ? min(x1, G - 1) : (x0 < 0 ? G - 1 : x1 - G);
-                    if (a > z1 || (part == 1 && x0 >= 0 && x1 < G)) continue;
+                    int a, z1;
+                    wrapped_run(x0, x1, G, part, &a, &z1);
+                    if (a > z1) continue;
                     const uint32_t e = start[rw + (uint32_t)z1 + 1];
                     for (uint32_t t = start[rw + (uint32_t)a]; t < e; ++t) {
                         const double4 c = cpos[t];
