@@ -60,6 +60,8 @@ template <> struct Th<float> {
     __device__ static float w(const DevParams& P, int r) { return P.w_f[r]; }
     __device__ static float half(const DevParams& P) { return P.half_f; }
     __device__ static float reach(const DevParams& P) { return P.s_reach_f; }
+    __device__ static float image(const DevParams& P) { return P.image_f; }
+    __device__ static float inv_image(const DevParams& P) { return P.inv_image_f; }
     __device__ static float vmax(const DevParams& P) { return P.vmax_f; }
     __device__ static float vmin(const DevParams& P) { return P.vmin_f; }
 };
@@ -70,6 +72,8 @@ template <> struct Th<double> {
     __device__ static double w(const DevParams& P, int r) { return P.w[r]; }
     __device__ static double half(const DevParams& P) { return P.half; }
     __device__ static double reach(const DevParams& P) { return P.s_reach; }
+    __device__ static double image(const DevParams& P) { return P.image; }
+    __device__ static double inv_image(const DevParams& P) { return P.inv_image; }
     __device__ static double vmax(const DevParams& P) { return P.vmax; }
     __device__ static double vmin(const DevParams& P) { return P.vmin; }
 };

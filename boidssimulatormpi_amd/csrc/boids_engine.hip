@@ -453,6 +453,16 @@ static int derive_thresholds(const bs_params* p, DevParams* P, std::string* why)
     P->s_reach_f = round_up_f(reach_f * reach_f);
     const double reach = (sqrt(P->s_max) + 1e-14 * p->field) * (1.0 + 1e-13);
     P->s_reach = reach * reach * (1.0 + 1e-15);
+    P->image_f = (float)p->field;
+    P->inv_image_f = 1.0f / P->image_f;
+    P->image = p->field;
+    P->inv_image = 1.0 / p->field;
+    // Where squares of the field's lengths leave the type's normal range (and
+    // their margins with them), every pair is a candidate: no filter.
+    const auto no_filter = [&](double limit) { return !(p->field > 1.0 / limit && p->field < limit); };
+    if (no_filter(1e15)) { P->s_reach_f = INFINITY; P->image_f = P->inv_image_f = 0.0f; }
+    if (no_filter(1e140)) { P->s_reach = INFINITY; P->image = P->inv_image = 0.0; }
+    P->reach_cells = -1.0f;
     P->band_k = 8.0f;   // >= 2*sqrt(3) lattice units of displacement error, x2 margin
     P->same_cone = 1;
     for (int k = 1; k < 3; ++k)
@@ -831,6 +841,8 @@ static int create_engine(const bs_params* fp, uint32_t count, bool batch, bs_eng
             const uint64_t half = 8ull * G * G * G;
             e->P.sx = e->prm.n <= (1u << 18) && half <= std::max<uint64_t>(8ull * e->prm.n, 1u << 15) ? 2 : 1;
             e->P.inv_edge = G / p->field;
+            if (isfinite(e->P.s_reach_f))
+                e->P.reach_cells = (float)(sqrt((double)e->P.s_reach_f) * e->P.sx * e->P.inv_edge);
             e->ncell1 = (uint32_t)((uint64_t)G * G * G * (e->P.sx == 2 ? 8 : 1) + 1);
         }
     }

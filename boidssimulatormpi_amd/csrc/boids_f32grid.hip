@@ -150,9 +150,10 @@ void k_f32_grid_wave(DevParams P, StateF32 in, StateF32 out, const float4* __res
     const int cx = (int)axis_cell((double)px, kc, G), cy = (int)axis_cell((double)py, kc, G),
               cz = (int)axis_cell((double)pz, kc, G);
     // some boid is not where its cell is (set while this launch runs if one it
-    // writes is not; either value will do then)
-    const bool all = __builtin_amdgcn_readfirstlane(
-                         (int)__hip_atomic_load(outside, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0;
+    // writes is not; either value will do then), or the field has no filter
+    const bool all = __builtin_amdgcn_readfirstlane((int)__hip_atomic_load(outside, __ATOMIC_RELAXED,
+                                                                           __HIP_MEMORY_SCOPE_AGENT)) != 0 ||
+                     P.reach_cells < 0.f;
 
     // Lane r: row r of the window, cells cx + x0 .. cx + x1 of it (unwrapped).
     // Ordinarily the (2 sub + 1)^2 rows within sub cells, each cut to the
@@ -168,7 +169,7 @@ void k_f32_grid_wave(DevParams P, StateF32 in, StateF32 out, const float4* __res
     if (!all) {
         // distance from the owner to the row's square of cells, in cells, and the
         // sphere's half-width there (margins of 1e-3 cells cover the rounding)
-        const float R = __builtin_amdgcn_sqrtf(P.s_reach_f) * inv_h + 1e-3f;
+        const float R = P.reach_cells + 1e-3f;
         const float fy = py * inv_h - (float)cy, fz = pz * inv_h - (float)cz, fx = px * inv_h - (float)cx;
         const float gy = fmaxf(fmaxf((float)dy - fy, fy - (float)(dy + 1)), 0.f);
         const float gz = fmaxf(fmaxf((float)dz - fz, fz - (float)(dz + 1)), 0.f);
@@ -214,7 +215,7 @@ void k_f32_grid_wave(DevParams P, StateF32 in, StateF32 out, const float4* __res
     // the boids within the largest radius will do ((3) decides exactly): the
     // minimum image is taken with one rounding (near2).  Each
     // batch's records are fetched while the previous batch is tested.
-    const float Ff = (float)P.F, inv_F = inv_h / (float)G, reach = reach_of(P, px, py, pz);
+    const float Ff = P.image_f, inv_F = P.inv_image_f, reach = reach_of(P, px, py, pz);
     auto record_of = [&](uint32_t m0) {
         const uint32_t m = min(m0 + lane, M - 1);
         // the last row k with excl[k] <= m (binary lifting over the lanes; rows

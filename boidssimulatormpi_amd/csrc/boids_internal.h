@@ -49,10 +49,12 @@ struct DevParams {
     double vmax, vmin;
     // float exact thresholds (reference-faithful float mode)
     float s_thr_f[3], c_thr_f[3], s_max_f;
-    // bounds that no pair within the largest radius reaches by the filters'
-    // one-rounding distance (boids_device.h: near2)
-    float s_reach_f;
-    double s_reach;
+    // the filters of the reference-order steps (boids_device.h: near2): bounds
+    // that no pair within the largest radius reaches by their one-rounding
+    // distance; the field edge and its inverse as they take them (0 where the
+    // filter lets every pair through); the bound in cells (float grid; < 0: none)
+    float s_reach_f, image_f, inv_image_f, reach_cells;
+    double s_reach, image, inv_image;
     float w_f[3];
     float vmax_f, vmin_f;
     int32_t cone[3];           // 1: the rule has a view cone (a < 1); 0: distance only

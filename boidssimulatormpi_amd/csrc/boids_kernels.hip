@@ -44,7 +44,7 @@ __global__ __launch_bounds__(kBlock) void k_allpairs_wave(DevParams P, St in, St
     uint32_t* near = list[wave];
     R px = in.x[i], py = in.y[i], pz = in.z[i], vx = in.vx[i], vy = in.vy[i], vz = in.vz[i];
     const R vn = norm3(vx, vy, vz);
-    const R reach = reach_of(P, px, py, pz), F = (R)P.F, inv_F = (R)1 / F;
+    const R reach = reach_of(P, px, py, pz), F = Th<R>::image(P), inv_F = Th<R>::inv_image(P);
     OrderedSums<R> S;
 
     // candidate positions two batches ahead of the one being tested
@@ -105,7 +105,7 @@ __global__ __launch_bounds__(kBlock) void k_allpairs_small(DevParams P, St in, S
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     R px = in.x[i], py = in.y[i], pz = in.z[i], vx = in.vx[i], vy = in.vy[i], vz = in.vz[i];
-    const R reach = reach_of(P, px, py, pz), F = (R)P.F, inv_F = (R)1 / F;
+    const R reach = reach_of(P, px, py, pz), F = Th<R>::image(P), inv_F = Th<R>::inv_image(P);
     const uint32_t batches = (n + 63) / 64;              // <= 64
     for (uint32_t b0 = wave; b0 < batches; b0 += 4 * kWaveOwners) {      // four batches' loads at once
         R x[4], y[4], z[4];

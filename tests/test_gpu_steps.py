@@ -165,3 +165,33 @@ def test_float_grid_at_the_largest_half_cells(n):
     assert all(np.array_equal(x, y) for x, y in zip(a.state_f32(), b.state_f32()))
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("F", [1e-3, 3e-15, 1e-16, 1e-19, 3e-23, 1e-39, 1e5, 3e14, 1e16, 1e19, 1e39])
+@pytest.mark.parametrize("mode", [E.MODE_ALLPAIRS_F32REF, E.MODE_GRID_F32REF, E.MODE_ALLPAIRS_F64])
+def test_fields_of_any_size(mode, F):
+    # fields whose squared lengths leave the floats' normal range are stepped without the candidate filter
+    n = 1500
+    print(mode, F, flush=True)
+    if mode == E.MODE_GRID_F32REF and F < 1e-20:
+        pytest.skip("squared distances underflow to 0: all-pairs then counts boids that no cell list meets")
+    if mode == E.MODE_ALLPAIRS_F64:
+        F = F ** 8 if 1e-39 < F < 1e39 else F                  # to 1e-184 and 1e152
+    rules = {k: (v[0] * F, *v[1:]) for k, v in RULES.items() if k[0] != "v"}
+    rules.update(vmax=0.005 * F, vmin=0.001 * F)
+    st = flock(n, False, n)
+    st[:, :3] = np.clip(st[:, :3], 0, 0.999)
+    with np.errstate(all="ignore"):
+        st = (st * F).astype(np.float32 if mode != E.MODE_ALLPAIRS_F64 else np.float64)
+        st = np.where(np.isfinite(st), st, 0).astype(st.dtype)
+        e = B.Engine(B.make_params(n, F, **rules, mode=mode, flags=E.FLAG_DIGEST))
+        assert e.info().mode == mode
+        p, v = st[:, :3].copy(), st[:, 3:].copy()
+        e.set_state(xyzv6=st) if st.dtype == np.float32 else e.set_state(pos=p, vel=v)
+        for t in range(2):
+            _, d = O.step(O.params(F, **rules), p, v, digest=True)
+            e.step(1)
+            gp, gv = e.state_f32() if st.dtype == np.float32 else e.state_f64()
+            assert np.array_equal(e.digest(), d), t
+            assert np.array_equal(gp, p, equal_nan=True) and np.array_equal(gv, v, equal_nan=True), t
+    e.close()
