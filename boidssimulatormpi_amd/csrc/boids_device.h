@@ -56,7 +56,6 @@ template <typename R> struct Th;
 template <> struct Th<float> {
     __device__ static float s(const DevParams& P, int r) { return P.s_thr_f[r]; }
     __device__ static float c(const DevParams& P, int r) { return P.c_thr_f[r]; }
-    __device__ static float smax(const DevParams& P) { return P.s_max_f; }
     __device__ static float w(const DevParams& P, int r) { return P.w_f[r]; }
     __device__ static float half(const DevParams& P) { return P.half_f; }
     __device__ static float reach(const DevParams& P) { return P.s_reach_f; }
@@ -68,7 +67,6 @@ template <> struct Th<float> {
 template <> struct Th<double> {
     __device__ static double s(const DevParams& P, int r) { return P.s_thr[r]; }
     __device__ static double c(const DevParams& P, int r) { return P.c_thr[r]; }
-    __device__ static double smax(const DevParams& P) { return P.s_max; }
     __device__ static double w(const DevParams& P, int r) { return P.w[r]; }
     __device__ static double half(const DevParams& P) { return P.half; }
     __device__ static double reach(const DevParams& P) { return P.s_reach; }

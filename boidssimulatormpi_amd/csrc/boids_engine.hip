@@ -1008,8 +1008,8 @@ static int grid_sort_into_a(bs_engine* e)
                                      e->start, e->db.id, e->perm, e->permid, e->stream));
     t2.stop();
     Timed t3(e, BS_K_GATHER);
-    HIP_TRY(e, launch_gather(flock_view(e), e->perm, e->permid, e->key, e->start, e->count, e->db, e->da,
-                             e->key_sorted, e->mode == BS_MODE_GRID_MIXED ? &e->lat : nullptr,
+    HIP_TRY(e, launch_gather(flock_view(e), e->perm, e->permid, e->key, e->start, e->db, e->da, e->key_sorted,
+                             e->mode == BS_MODE_GRID_MIXED ? &e->lat : nullptr,
                              e->mode == BS_MODE_GRID_F64 ? e->rec : nullptr, e->stream));
     t3.stop();
     return BS_OK;

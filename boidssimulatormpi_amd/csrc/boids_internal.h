@@ -145,8 +145,8 @@ hipError_t launch_scatter_ranked(Flocks F, Rows R, int max_cols, uint32_t* row_o
 // lat (mixed) receives the lattice copy; rec (FP64 grid) the records the
 // neighbour kernel fetches, three planes of n double2: (x, y), (z, vx), (vy, vz).
 hipError_t launch_gather(Flocks F, const uint32_t* perm, const uint32_t* permid, const uint32_t* key,
-                         const uint32_t* start, uint32_t* count, StateF64 src, StateF64 dst,
-                         uint32_t* key_sorted, Lattice* lat, double2* rec, hipStream_t stream);
+                         const uint32_t* start, StateF64 src, StateF64 dst, uint32_t* key_sorted, Lattice* lat,
+                         double2* rec, hipStream_t stream);
 // Neighbour kernels (boids_nbr.hip).  nb = workgroup size (64, 128 or 256),
 // tile = LDS candidates per thread and pass (5, 6, 9 or 12), max_cols = most x
 // columns of a chunk's tile (columns a chunk covers + 2 sx), max_chunks =

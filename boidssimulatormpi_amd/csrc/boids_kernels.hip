@@ -22,11 +22,12 @@ namespace boids {
 // append those below it to an LDS list, in ascending j -- the reference's
 // summation order (src/boid_simulation.cpp:153-212); whenever it holds 64, they
 // go through OrderedSums (src/boid_simulation.cpp:216-248 after the last).
-// R = float: bit-identical to boidsim.  R = double: the FP64 promotion.  A flock
-// of N boids takes N waves, so small flocks (N = 1024) still fill the chip, a
-// wave per SIMD: what bounds them is one wave's chain.
-// One update: float N = 1000 20.1 us (21.2 with every candidate decided exactly
-// and the terms handed round by lane reads), FP64 N = 1024 11.9 us (12.5).
+// R = float: bit-identical to boidsim.  R = double: the FP64 promotion.  For
+// flocks above 4096 boids (double: 3072), which fill the chip with a wave per
+// boid; what bounds it is the tests of the candidates, and in crowded flocks the
+// ordered sums.  One update of N = 8192, uniform / all in reach of all, with the
+// synchronisation: float 82 / 524 us, FP64 141 / 747 (170 / 5816 and 204 / 7284
+// with every candidate decided exactly and the terms handed round by lane reads).
 // ---------------------------------------------------------------------------
 constexpr int kWaveOwners = kBlock / 64;     // owners (waves) per workgroup
 
@@ -482,8 +483,7 @@ __global__ __launch_bounds__(kBlock) void k_sort_runs(Flocks F, Rows R, const ui
 // the search measured slower: its loop is as long as the part).
 __global__ __launch_bounds__(kBlock) void k_gather(Flocks F, const uint32_t* perm,
                                                    const uint32_t* permid, const uint32_t* key,
-                                                   const uint32_t* start, uint32_t* count,
-                                                   StateF64 src, StateF64 dst,
+                                                   const uint32_t* start, StateF64 src, StateF64 dst,
                                                    uint32_t* key_sorted, Lattice lat, int with_lat,
                                                    double2* rec)
 {
@@ -507,7 +507,6 @@ __global__ __launch_bounds__(kBlock) void k_gather(Flocks F, const uint32_t* per
     dst.vx[f] = vx; dst.vy[f] = vy; dst.vz[f] = vz;
     dst.id[f] = me;
     key_sorted[f] = c;
-    if (rank == 0) count[c] = 0u;
     if (with_lat) {
         const DevParams& P = F.fl[flock_of(F, f)].P;   // slots stay inside their flock
         const double scale = P.lat_scale;
@@ -661,13 +660,13 @@ hipError_t launch_scatter_ranked(Flocks F, Rows R, int max_cols, uint32_t* row_o
 }
 
 hipError_t launch_gather(Flocks F, const uint32_t* perm, const uint32_t* permid, const uint32_t* key,
-                         const uint32_t* start, uint32_t* count, StateF64 src, StateF64 dst,
-                         uint32_t* key_sorted, Lattice* lat, double2* rec, hipStream_t stream)
+                         const uint32_t* start, StateF64 src, StateF64 dst, uint32_t* key_sorted, Lattice* lat,
+                         double2* rec, hipStream_t stream)
 {
     if (F.n == 0) return hipSuccess;
     Lattice l = lat ? *lat : Lattice{nullptr, nullptr};
     hipLaunchKernelGGL(k_gather, dim3(blocks_for(F.n)), dim3(kBlock), 0, stream, F, perm, permid,
-                       key, start, count, src, dst, key_sorted, l, lat ? 1 : 0, rec);
+                       key, start, src, dst, key_sorted, l, lat ? 1 : 0, rec);
     return hipGetLastError();
 }
 

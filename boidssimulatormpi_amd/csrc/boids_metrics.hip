@@ -7,10 +7,8 @@
 // Input: n positions / velocities in id order (double, AoS x,y,z).  A private
 // uniform grid (edge >= eps, >= 3 cells per axis when possible, about one
 // boid per cell at most) is built with the engine's scan; the searches run
-// over the cell-ordered copy, one boid per lane, so a wave's lanes sit in
-// neighbouring cells and read the same candidates.  Latency is what bounds
-// them (131072 boids are two waves per SIMD): the nine rows' cell starts are
-// read together, and a row's three cells are one run of slots.
+// over the cell-ordered copy, four lanes per boid (k_m_near), so a wave's 16
+// boids sit in neighbouring cells and read the same candidates.
 #include "boids_internal.h"
 
 #include <math.h>
