@@ -12,6 +12,8 @@
  *     bs_last_error() then describes the failure.  (The reference prints to
  *     std::cerr and calls exit(-1); the C++ shim maps errors back to that.)
  *   - One host thread per engine; calls on one engine must not overlap.
+ *   - A call works on the engine's device and leaves the caller's current
+ *     device as it was (bs_create leaves the engine's current).
  *   - Host arrays are in boid-id order (the order get(id, ...) uses).
  *   - Modes: see BS_MODE_*.  All GPU work is hand-written HIP for gfx950.
  */
@@ -107,7 +109,8 @@ typedef struct {
     int32_t mode;                /* effective mode (grid modes may fall back to all-pairs) */
     int32_t cells_per_axis;      /* 0 for all-pairs */
     double cell_edge;
-    uint64_t device_bytes;       /* device memory the engine holds */
+    uint64_t device_bytes;       /* device memory the engine holds (not the library's pinned host
+                                  * staging: at most 4 buffers of up to 16 MiB while an engine lives) */
     uint64_t steps;              /* updates done since the last set_state/init */
     int32_t block;               /* neighbour-kernel workgroup size (grid modes), else 0 */
     int32_t tile;                /* LDS tile depth (grid modes), else 0 */

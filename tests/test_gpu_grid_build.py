@@ -112,10 +112,9 @@ def test_cells_per_axis_is_the_exact_cube_root_cap():
 @pytest.mark.parametrize("mode", [E.MODE_GRID_F64, E.MODE_GRID_MIXED])
 def test_grid_build_crowded_cells_span_sort_windows(mode):
     # cells of 3000, 1500, 700, 100, 65 and 64 boids (ids drawn at random):
-    # a cell of more than 64 boids takes its in-cell id order from 1024-slot
-    # sorted windows merged by binary search, a smaller one from a pass over
-    # its ids; a cell spanning three or four windows must still come out in
-    # ascending id order
+    # a cell takes its in-cell id order from its parts in the runs of 64 slots,
+    # each sorted, merged by binary search; a cell spanning many runs must
+    # still come out in ascending id order
     n, F = 1 << 16, 1.0
     rng = np.random.default_rng(11)
     st = B.generate_init(E.INIT_RANDOM_UNIFORM, n, F, CFG0["vmax"], CFG0["vmin"], seed=5)

@@ -196,7 +196,7 @@ def test_f32_grid_crowded_owners_and_oracle():
     # Two crowded cubes of edge 0.01 (every pair inside a cube lies within
     # every radius).  Cube A holds 1500 boids: each of their owners has 1499
     # boids within the largest radius, more than the per-wave sorted list
-    # holds (1024), and takes the serial 27-way merge.  Cube B holds 900:
+    # holds (1024), and takes them in windows of ascending ids.  Cube B holds 900:
     # their owners sort lists of ~900 ids (1024 with the padding).  Everyone
     # else sorts short lists.  All must equal the float all-pairs step and the
     # float oracle.
