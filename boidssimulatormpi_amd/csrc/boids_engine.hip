@@ -1021,9 +1021,9 @@ static int grid_sort_into_a(bs_engine* e)
 //     while the next is under way.  In, parts of kInPart (10^4 boids 137 -> 60 us,
 //     130000 boids 608 -> 190 us).  Out, one part up to 2 kOutPart and then equal
 //     ones of about kOutPart, 6 at most: a part of its own costs about 12 us, the
-//     copy on the host it hides about 40 us a MB (FP64 states after an update:
-//     16384 boids 193 us before, 163 in parts of 256 KB, 124 this way; 50021 321,
-//     270, 237; 116000 528, 384, 379);
+//     copy on the host that it hides 20 to 40 us a MB (FP64 states after an
+//     update: 16384 boids 193 us before, 163 in parts of 256 KB, 124 this way;
+//     50021 321, 270, 237; 116000 528, 384, 379);
 //   above it: in pieces of kPiece that up to kStageThreads threads carry, each
 //     through a piece of the staging of its own, so the copies to and from
 //     the caller's pages (a few GB/s a thread, page faults included) run
